@@ -36,6 +36,22 @@ int sidon_res_norm(float* x, const float* y, const float* bias, const float* n1_
                    int xn_fp16, int R, int C, sidon_stream_t stream);
 
 /*
+ * The same at the end of a residual projection whose K range was split
+ * (sidon_gemm_part): the partial sums part [splits, R, C] fp32 join the
+ * stream here instead of in a pass of their own.
+ *
+ *   x_r  = x_r + sum over s of part[s, r]     in the order s = 0, 1, ...
+ *   n1_w == NULL:  x_r is stored back;  xn_r = LN2(x_r + bias)
+ *   n1_w != NULL:  x_r = LN1(x_r + bias) is stored back;  xn_r = LN2(x_r)
+ *
+ * xn [R, C] fp16 if n2_w != NULL, else nothing but x is written; bias may be
+ * NULL.  splits in [1, 8]; C, types and alignment as for sidon_res_norm.
+ */
+int sidon_res_norm_parts(float* x, const float* part, int splits, const float* bias, const float* n1_w,
+                         const float* n1_b, float eps1, const float* n2_w, const float* n2_b, float eps2, void* xn,
+                         int R, int C, sidon_stream_t stream);
+
+/*
  * GLU of the pointwise conv's output: g[r, c] = h[r, c] * sigmoid(h[r, C + c])
  * for h [R, 2C] and g [R, C] fp16 (row-major, contiguous), math in fp32.
  * Replaces glu / _glu_kernel of src/sidon_triton/triton_encoder.py:113-133.
@@ -64,8 +80,8 @@ int sidon_silu(void* h, int64_t n, sidon_stream_t stream);
  * sidon_gemm_bias_act_fits(M, N, K) says whether a shape is supported (pure
  * host function); sidon_gemm_bias_act_preferred(M, N, K) whether the kernel
  * is expected to beat a library GEMM followed by sidon_silu on the current
- * device (its 320 x 256 tiles keep >= 3/4 of the CUs busy in every round).
- * Neither has a counterpart in the reference.
+ * device, and sidon_gemm_lt_act (its 320 x 256 tiles keep >= 4/5 of the CUs
+ * busy in every round).  Neither has a counterpart in the reference.
  */
 int sidon_gemm_bias_act_fits(int M, int N, int K);
 int sidon_gemm_bias_act_preferred(int M, int N, int K);
@@ -85,13 +101,31 @@ int sidon_gemm_bias_act(const void* x, int ldx, const void* w, int ldw, const vo
  * before the SiLU: the two differ by at most about one fp16 ulp).  Replaces
  * the torch.addmm(b1, xn, W1^T) + in-place F.silu pair of
  * src/sidon_triton/triton_encoder.py:498-499 and :507-508.  Shapes: M, N,
- * K >= 1, strides >= the row lengths, every operand 2-byte aligned.  The
- * kernel is hipBLASLt's first heuristic choice that needs no workspace,
- * kept per problem; the first call on a device creates its hipBLASLt handle
- * and must not run during stream capture.
+ * K >= 1, strides >= the row lengths, every operand 2-byte aligned.  Where
+ * sidon_gemm_half_preferred(M, N, K) (N and K multiples of 64, up to 9 * 2^20
+ * outputs) and the operands are 16-byte aligned with strides that are
+ * multiples of 8, this library's own kernel runs with the same rounding.
+ * Elsewhere the kernel is hipBLASLt's first heuristic choice that needs no
+ * workspace, kept per problem, and the first call on a device creates its
+ * hipBLASLt handle and must not run during stream capture.
  */
+int sidon_gemm_half_preferred(int M, int N, int K);
 int sidon_gemm_lt_act(const void* x, int ldx, const void* w, int ldw, const void* bias, void* y, int ldy, int M,
                       int N, int K, int act, sidon_stream_t stream);
+
+/*
+ * The pointwise conv's first projection with the GLU in its epilogue:
+ *
+ *   y[m, c] = a . sigmoid(b),  a = x[m, :] . w[c, :],  b = x[m, :] . w[C + c, :]
+ *
+ * with a and b rounded to fp16 first (as a separate GEMM stores them) and the
+ * GLU in fp32, rounded to fp16 as sidon_glu does.  x [M, K] and w [2 C, K]
+ * fp16 (K contiguous), y [M, C] fp16; C a multiple of 32, K of 64; strides
+ * multiples of 8, operands 16-byte aligned, y apart from x and w.  Replaces
+ * the F.linear + glu of src/sidon_triton/triton_encoder.py:504-505.
+ */
+int sidon_gemm_glu(const void* x, int ldx, const void* w, int ldw, void* y, int ldy, int M, int C, int K,
+                   sidon_stream_t stream);
 
 /*
  * Residual projection, accumulated into the fp32 stream in place:
@@ -101,21 +135,39 @@ int sidon_gemm_lt_act(const void* x, int ldx, const void* w, int ldw, const void
  * x [M, K] and w [N, K] fp16 row-major (K contiguous: activations and a torch
  * Linear weight), y [M, N] fp32 row-major, updated in place.  Replaces the
  * torch.addmm(x, a, w.t(), out_dtype=torch.float32, out=x) of res(),
- * src/sidon_triton/triton_encoder.py:491-492.  64 x 64 output tiles, K split
- * over the workgroup's 4 wavefronts and summed in a fixed order: the result
- * does not depend on timing.  Shapes: M >= 1, N a multiple of 64, K a
+ * src/sidon_triton/triton_encoder.py:491-492.  Every output is summed over K in
+ * order by one wavefront: the result does not depend on timing.  Shapes: M >= 1, N a multiple of 64, K a
  * multiple of 128; ldx, ldw multiples of 8 and >= K, ldy a multiple of 4 and
  * >= N; x, w, y 16-byte aligned; x and w must not overlap y (checked on the byte ranges
  * the call touches: SIDON_E_SHAPE).  sidon_gemm_res_fits(M, N, K) says whether
  * a shape is supported (pure host function); sidon_gemm_res_preferred(M, N,
- * K) whether the kernel is expected to beat a library GEMM on the current
- * device (its tiles fit one per compute unit).  Neither has a counterpart in
+ * K) whether it, or sidon_gemm_part, is expected to beat a library GEMM on
+ * the current device (up to 5 * 2^20 outputs).  Neither has a counterpart in
  * the reference.
  */
 int sidon_gemm_res_fits(int M, int N, int K);
 int sidon_gemm_res_preferred(int M, int N, int K);
 int sidon_gemm_res(const void* x, int ldx, const void* w, int ldw, float* y, int ldy, int M, int N, int K,
                    sidon_stream_t stream);
+
+/*
+ * The same projection with its K range split over workgroups:
+ *
+ *   part[s, m, n] = sum over the s-th K range of x[m, k] w[n, k]
+ *
+ * for sidon_res_norm_parts to add to the stream, so that a short chunk's few
+ * output tiles still fill the chip.  Shapes, strides and alignment of x and w
+ * as for sidon_gemm_res.  sidon_gemm_part_splits(M, N, K): the number of K
+ * ranges (1 to 8; 1 means that sidon_gemm_res is the better call; 0 for an
+ * unsupported shape); a function of the shape and the device alone.
+ * part: part_elems >= splits * M * N fp32 values, 16-byte aligned, apart from
+ * x and w; for every call of up to M rows sidon_gemm_part_rows(M) * N values
+ * are enough (pure host function).  No counterpart in the reference.
+ */
+int sidon_gemm_part_splits(int M, int N, int K);
+int64_t sidon_gemm_part_rows(int M);
+int sidon_gemm_part(const void* x, int ldx, const void* w, int ldw, float* part, int64_t part_elems, int M, int N,
+                    int K, sidon_stream_t stream);
 
 /*
  * Plain GEMM on rocBLAS with the kernel chosen per problem by timing:

@@ -37,6 +37,8 @@ SIGNATURES = {
     "sidon_flexrel_debug_rerun_all": (None, [ctypes.c_int]),
     "sidon_res_norm": (ctypes.c_int, [_VP, _VP, _VP, _VP, _VP, ctypes.c_float, ctypes.c_int, _VP, _VP,
                                       ctypes.c_float, _VP, ctypes.c_int, ctypes.c_int, ctypes.c_int, _VP]),
+    "sidon_res_norm_parts": (ctypes.c_int, [_VP, _VP, ctypes.c_int, _VP, _VP, _VP, ctypes.c_float, _VP, _VP,
+                                            ctypes.c_float, _VP, ctypes.c_int, ctypes.c_int, _VP]),
     "sidon_glu": (ctypes.c_int, [_VP, _VP, ctypes.c_int, ctypes.c_int, _VP]),
     "sidon_silu": (ctypes.c_int, [_VP, ctypes.c_int64, _VP]),
     "sidon_gemm_bias_act_fits": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
@@ -45,6 +47,13 @@ SIGNATURES = {
                                            ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _VP]),
     "sidon_gemm_lt_act": (ctypes.c_int, [_VP, ctypes.c_int, _VP, ctypes.c_int, _VP, _VP, ctypes.c_int,
                                          ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _VP]),
+    "sidon_gemm_half_preferred": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "sidon_gemm_glu": (ctypes.c_int, [_VP, ctypes.c_int, _VP, ctypes.c_int, _VP, ctypes.c_int, ctypes.c_int,
+                                      ctypes.c_int, ctypes.c_int, _VP]),
+    "sidon_gemm_part_splits": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "sidon_gemm_part_rows": (ctypes.c_int64, [ctypes.c_int]),
+    "sidon_gemm_part": (ctypes.c_int, [_VP, ctypes.c_int, _VP, ctypes.c_int, _VP, ctypes.c_int64, ctypes.c_int,
+                                       ctypes.c_int, ctypes.c_int, _VP]),
     "sidon_gemm_res_fits": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "sidon_gemm_res_preferred": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "sidon_gemm_res": (ctypes.c_int, [_VP, ctypes.c_int, _VP, ctypes.c_int, _VP, ctypes.c_int, ctypes.c_int,

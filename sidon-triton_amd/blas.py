@@ -7,13 +7,13 @@ type combinations:
   * fp32 x, w, out -- the framing matmul of the front end
     (src/sidon_triton/frontend.py:222);
   * fp16 x, w, out (beta 0) -- the pointwise conv's first F.linear
-    (src/sidon_triton/triton_encoder.py:504);
+    (src/sidon_triton/triton_encoder.py:504) at widths that
+    ``conformer.linear_glu`` does not take;
   * fp16 x, w and an fp32 out, beta 1 -- the form of the residual projections
     of res(), ``torch.addmm(x, a, W^T, out_dtype=float32, out=x)`` (:491-492).
-    The encoder does not use rocBLAS for those: inside its graph rocBLAS's
-    timed choice measured no faster (feed-forward output) or slower (the
-    hidden -> hidden projections) than torch.addmm, which it keeps for long
-    chunks, and short chunks take ``conformer.residual_gemm``.
+    The encoder does not use rocBLAS for those: they run on this library's
+    tiled kernel (``conformer.residual_partials`` / ``residual_gemm``), which
+    measured faster.
 
 The first call of a problem (shape, strides, types, beta != 0) on a device,
 made while the stream is not capturing, times rocBLAS's kernels for it on

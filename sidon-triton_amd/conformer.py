@@ -11,6 +11,11 @@ Same names and argument meaning as src/sidon_triton/triton_encoder.py:
     summation order; csrc/gemm.hip), for the shapes ``linear_silu_fits``
     accepts (N a multiple of 256, K of 64);
 
+  * ``linear(x, w, b, out)`` and ``linear_glu(x, w)``: the plain projections
+    and the pointwise conv's with its GLU (:500-505);
+  * ``residual_gemm`` / ``residual_partials``: the projections into the fp32
+    stream (:491-492), in place or as partial sums for the next norm;
+
 plus ``glu_causal_dw_norm(h, ...)``, the two fused: it reads the pointwise
 conv's output h [B*T, 2C] and forms g on the fly (bit-identical to
 ``causal_dw_norm(glu(h), ...)``, without the g round trip through HBM).
@@ -118,9 +123,10 @@ def linear_silu_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def linear_silu_preferred(rows: int, n: int, k: int, device=None) -> bool:
-    """Whether ``linear_silu`` is expected to beat ``silu_(torch.addmm(...))``
-    for x [rows, k], w [n, k] on ``device`` (its tiles fill >= 3/4 of the CUs
-    in every round; at n = 4096, k = 1024 that is rows > 3840 on 256 CUs)."""
+    """Whether ``linear_silu`` is expected to beat ``linear_silu_lt`` and
+    ``silu_(torch.addmm(...))`` for x [rows, k], w [n, k] on ``device`` (past
+    ``linear_silu_lt``'s own kernel, where 320 x 256 tiles fill >= 4/5 of the
+    CUs in every round; at n = 4096, k = 1024 that is rows > 3840 on 256 CUs)."""
     with torch.cuda.device(device):
         return bool(_lib.load().sidon_gemm_bias_act_preferred(rows, n, k))
 
@@ -165,11 +171,12 @@ def linear_silu(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, out: t
 
 def linear_silu_lt(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, out: torch.Tensor | None = None,
                    act: bool = True) -> torch.Tensor:
-    """silu(x . w^T + b) [M, N] fp16 on hipBLASLt with the bias and SiLU in
-    its epilogue (fp32 sum + bias, SiLU in fp32, one rounding to fp16), for
+    """silu(x . w^T + b) [M, N] fp16 with the bias and SiLU in the GEMM's
+    epilogue (fp32 sum + bias, SiLU in fp32, one rounding to fp16), for
     x [M, K] and w [N, K] fp16 (rows K-contiguous), b [N] fp16 or None;
-    act=False leaves out the SiLU.  The first call on a device must not run
-    during stream capture."""
+    act=False leaves out the SiLU.  On this library's tiled kernel where
+    ``sidon_gemm_half_preferred`` and the alignment allow, else on hipBLASLt,
+    whose first call on a device must not run during stream capture."""
     device = x.device
     rows, n, k, out = _linear_args(x, w, b, out)
     lib = _lib.load()
@@ -181,6 +188,49 @@ def linear_silu_lt(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, out
     return out
 
 
+def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+    """out = x . w^T + b, fp16 with fp32 sums: this library's GEMM kernel up to
+    the sizes where it beats the library (``sidon_gemm_half_preferred``), else
+    torch.addmm.  x [M, K], w [N, K], out [M, N]."""
+    with torch.cuda.device(x.device):
+        own = _lib.load().sidon_gemm_half_preferred(x.shape[0], w.shape[0], w.shape[1])
+    if own:
+        return linear_silu_lt(x, w, b, out=out, act=False)
+    return torch.addmm(b, x, w.t(), out=out)
+
+
+def linear_glu_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether ``linear_glu`` takes x [M, K] and w [2C, K]."""
+    return w.shape[0] % 64 == 0 and w.shape[1] % 64 == 0 and x.shape[1] == w.shape[1]
+
+
+def linear_glu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+    """``glu(x . w^T)`` in one kernel (src/sidon_triton/triton_encoder.py:504-505):
+    x [M, K] and w [2C, K] fp16 with K contiguous -> [M, C] fp16, the products
+    rounded to fp16 in front of the GLU as a separate GEMM stores them."""
+    device = x.device
+    for name, t in (("x", x), ("w", w)):
+        _check_device_tensor(name, t, device)
+        if t.dtype != torch.float16 or t.dim() != 2 or t.stride(1) != 1:
+            raise ValueError(f"{name} must be a float16 [rows, K] tensor with K contiguous")
+    rows, k = x.shape
+    if w.shape[1] != k or w.shape[0] % 2:
+        raise ValueError(f"x is {tuple(x.shape)}, w {tuple(w.shape)}")
+    c = w.shape[0] // 2
+    if out is None:
+        out = torch.empty(rows, c, device=device, dtype=torch.float16)
+    else:
+        _check_device_tensor("out", out, device)
+        if out.dtype != torch.float16 or tuple(out.shape) != (rows, c) or out.stride(1) != 1:
+            raise ValueError(f"out must be a float16 [{rows}, {c}] tensor with rows contiguous")
+    lib = _lib.load()
+    with torch.cuda.device(device):
+        rc = lib.sidon_gemm_glu(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
+                                rows, c, k, _stream_handle(device))
+    _lib.check("sidon_gemm_glu", rc)
+    return out
+
+
 def residual_gemm_fits(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``residual_gemm`` takes a [M, K], w [N, K] into x [M, N]."""
     return (bool(_lib.load().sidon_gemm_res_fits(a.shape[0], w.shape[0], w.shape[1])) and a.shape[1] == w.shape[1]
@@ -189,32 +239,82 @@ def residual_gemm_fits(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> boo
 
 def residual_gemm_preferred(rows: int, n: int, k: int, device=None) -> bool:
     """Whether ``residual_gemm`` is expected to beat torch.addmm for a
-    [rows, k], w [n, k] on ``device`` (its 64 x 64 tiles fit one per compute
-    unit: rows <= 1024 at n = 1024 on 256 CUs)."""
+    [rows, k], w [n, k] on ``device`` (up to 5 * 2^20 outputs)."""
     with torch.cuda.device(device):
         return bool(_lib.load().sidon_gemm_res_preferred(rows, n, k))
+
+
+def residual_splits(rows: int, n: int, k: int, device=None) -> int:
+    """K ranges of ``residual_partials`` for a [rows, k], w [n, k]: 2 to 8, or 1
+    where the in-place ``residual_gemm`` is the better call, or 0 where
+    torch.addmm is.  Depends on the shape and the device alone."""
+    lib = _lib.load()
+    with torch.cuda.device(device):
+        return int(lib.sidon_gemm_part_splits(rows, n, k)) if lib.sidon_gemm_res_preferred(rows, n, k) else 0
+
+
+def partial_values(rows: int, n: int) -> int:
+    """fp32 values that hold the partial sums of any call of up to ``rows`` rows."""
+    return int(_lib.load().sidon_gemm_part_rows(rows)) * n
+
+
+def _residual_operands(a: torch.Tensor, w: torch.Tensor, device: torch.device):
+    for name, t in (("a", a), ("w", w)):
+        _check_device_tensor(name, t, device)
+        if t.dtype != torch.float16 or t.dim() != 2 or t.stride(1) != 1:
+            raise ValueError(f"{name} must be a float16 [rows, K] tensor with K contiguous")
+    if w.shape[1] != a.shape[1]:
+        raise ValueError(f"a has {a.shape[1]} columns, w {w.shape[1]}")
+    return a.shape[0], w.shape[0], a.shape[1]
+
+
+def residual_partials(a: torch.Tensor, w: torch.Tensor, part: torch.Tensor) -> torch.Tensor:
+    """a . w^T [M, N] as partial sums over ``residual_splits`` K ranges, for
+    ``encoder_block.res_norm_parts`` to add to the stream: a [M, K] and w [N, K]
+    fp16 with K contiguous, part a contiguous fp32 buffer (``partial_values``).
+    Returns the [splits, M, N] view of ``part`` that holds them."""
+    device = a.device
+    rows, n, k = _residual_operands(a, w, device)
+    _check_device_tensor("part", part, device)
+    if part.dtype != torch.float32 or not part.is_contiguous():
+        raise ValueError("part must be a contiguous float32 tensor")
+    lib = _lib.load()
+    with torch.cuda.device(device):
+        splits = lib.sidon_gemm_part_splits(rows, n, k)
+        rc = lib.sidon_gemm_part(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), part.data_ptr(), part.numel(),
+                                 rows, n, k, _stream_handle(device))
+    _lib.check("sidon_gemm_part", rc)
+    return part.view(-1)[:splits * rows * n].view(splits, rows, n)
 
 
 def residual_gemm(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x += a . w^T in place: x [M, N] fp32 (the residual stream), a [M, K]
     and w [N, K] fp16 with K contiguous -- the
     ``torch.addmm(x, a, w.t(), out_dtype=torch.float32, out=x)`` of the
-    reference's res() (src/sidon_triton/triton_encoder.py:491-492)."""
+    reference's res() (src/sidon_triton/triton_encoder.py:491-492).  Short
+    streams with contiguous rows take K split over workgroups and a pass that
+    adds the partial sums (allocated per call); the sums are taken in a fixed
+    order either way."""
     device = x.device
-    for name, t in (("a", a), ("w", w)):
-        _check_device_tensor(name, t, device)
-        if t.dtype != torch.float16 or t.dim() != 2 or t.stride(1) != 1:
-            raise ValueError(f"{name} must be a float16 [rows, K] tensor with K contiguous")
+    rows, n, k = _residual_operands(a, w, device)
     _check_device_tensor("x", x, device)
-    rows, k = a.shape
-    n = w.shape[0]
-    if w.shape[1] != k:
-        raise ValueError(f"a has {k} columns, w {w.shape[1]}")
     if x.dtype != torch.float32 or tuple(x.shape) != (rows, n) or x.stride(1) != 1:
         raise ValueError(f"x must be a float32 [{rows}, {n}] tensor with rows contiguous")
     lib = _lib.load()
     with torch.cuda.device(device):
+        stream = _stream_handle(device)
+        # The pass that adds the partial sums (2-3 us) pays only for a long K.
+        splits = lib.sidon_gemm_part_splits(rows, n, k) if x.is_contiguous() and k >= 2 * n and n <= 2048 else 1
+        if splits > 1 and x.data_ptr() % 16 == 0:
+            part = torch.empty(splits * rows * n, device=device)
+            rc = lib.sidon_gemm_part(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), part.data_ptr(),
+                                     part.numel(), rows, n, k, stream)
+            _lib.check("sidon_gemm_part", rc)
+            rc = lib.sidon_res_norm_parts(x.data_ptr(), part.data_ptr(), splits, None, None, None, 0.0, None, None,
+                                          0.0, None, rows, n, stream)
+            _lib.check("sidon_res_norm_parts", rc)
+            return x
         rc = lib.sidon_gemm_res(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), x.data_ptr(), x.stride(0),
-                                rows, n, k, _stream_handle(device))
+                                rows, n, k, stream)
     _lib.check("sidon_gemm_res", rc)
     return x

@@ -1,309 +1,220 @@
-// gemm.hip -- the conformer FFN's input projection with its bias and SiLU
-// fused, for MI355X (gfx950).
+// gemm.hip -- the encoder's fp16 projections on the tiled GEMM kernel of
+// gemm_tile.h (MI355X / gfx950): the host side that checks arguments, picks
+// the tile shape and the K split, and launches.
 //
-//   Y[m, n] = act(X[m, :] . W[n, :] + bias[n])        act = SiLU or identity
+//   sidon_gemm_bias_act   y = act(fp16(x . w^T + bias))            feed-forward input, two roundings
+//   sidon_gemm_lt_act     y = act(x . w^T + bias), one rounding    (blaslt.hip calls gemm_half below)
+//   sidon_gemm_glu        y = a . sigmoid(b), (a | b) = x . w^T    pointwise conv 1 + GLU
+//   sidon_gemm_res        y += x . w^T, fp32 in place              residual projections
+//   sidon_gemm_part       partial sums of x . w^T, K split         the same, summed by the next norm
 //
-// X [M, K] and W [N, K] fp16 (both K-contiguous: activations and a torch
-// Linear weight), fp32 accumulation, Y [M, N] fp16.  This is the
-// torch.addmm(b1, xn, W1^T) + F.silu_ pair of the FFN modules of
-// src/sidon_triton/triton_encoder.py:498-499 and :507-508, in one pass: the
-// bias is added to the fp32 sum and rounded to fp16 (as the addmm stores it),
-// then SiLU is taken in fp32 and rounded to fp16 (as the in-place SiLU does),
-// so the only difference from the two-step form is the GEMM's summation order.
+// These are the GEMMs of src/sidon_triton/triton_encoder.py:491-510 (with the
+// F.silu_ of :499 / :508 and the GLU of :505 taken in the epilogue).
 //
-// Tiling.  A workgroup owns a 320 x 256 tile of Y and runs 8 wavefronts (two
-// per SIMD), wavefront (wm, wn) owning rows 160 wm + [0, 160) and columns
-// 64 wn + [0, 64) as 5 x 2 blocks of v_mfma_f32_32x32x16_f16 (Y^T = W . X^T,
-// so a lane holds four consecutive columns of one row).  The K loop walks
-// 64-wide slices: X and W slices (40 KB + 32 KB) are copied global -> LDS
-// with global_load_lds_dwordx4 into one of two buffers while the other is
-// consumed; one barrier per slice.  The operands of each k16 step are read
-// from LDS while the previous step's 10 MFMAs run.  16-byte chunk c of the
-// 128-byte LDS row r sits at chunk c ^ ((r >> 1) & 7), so the operand reads
-// (16 rows per 16 lanes) are bank-conflict free.  The epilogue stages each
-// wavefront's 160 x 64 fp16 result in LDS and writes whole 128-byte row
-// segments.  At M = 4800, N = 4096 the 240 tiles fill 240 CUs in one round.
-#include <hip/hip_runtime.h>
-
-#include <stdint.h>
+// Tile choice.  A launch of n tiles takes about
+//
+//   3.0 + load (0.062 nk mm + 0.031 nk + e mm) + 0.065 (n / CUs) nk cp   us
+//
+// with load = ceil(n / CUs) tiles on the busiest CU, nk 64-wide K slices per
+// tile, mm = BM BN / 4096 its MFMA work, cp = (BM + BN) / 64 its copy
+// traffic and e = 0.39 (fp16 out) or 0.48 (fp32 out): fitted to 1400 timings
+// of the encoder's five projections at M = 25-4800 with weights from HBM
+// (rms 9%).  The tile with the least estimate is taken; it is 0-3% (mean per
+// projection) slower than the best one measured.  A K split costs the norm
+// behind it its partial tiles and the stream's write on top, out of the MALL
+// (4 splits at M = 750: 0.7 us for 15 MB).
+//
+// Measured on MI355X (weights from HBM, graph replays, us), own | library:
+//   M =                          150          750          1600         4800
+//   4096 x 1024 + bias + SiLU    7.5 | 12.0+  12.3 | 14.3+ 20.4 | 22.3+ 47.0 | 47.0+  (library without SiLU)
+//   3072 x 1024 + bias           6.2 |  9.7    9.7 | 12.8  15.0 | 17.7  35.4 | 30.9
+//   2048 x 1024 + GLU            5.3 |  8.6+   6.8 |  9.7+ 10.3 | 13.2+ 23.3 | 30.6+  (library without GLU)
+//   1024 x 4096 fp32, split K    6.2 | 12.2   12.3 | 20.8  20.4 | 28.8  45.1 | 50.6
+//   1024 x 1024 fp32, split K    4.0 |  8.2    5.6 |  9.2   7.8 | 11.0  14.6 | 19.1
+#include "gemm_tile.h"
 
 #include "sidon_encoder.h"
 #include "sidon_host.h"
 
 #define SIDON_API extern "C" __attribute__((visibility("default")))
-#define SIDON_INLINE __attribute__((always_inline))
 
 namespace {
 
-typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+using namespace sidon_gemm;
+using sidon::fail;
 
-constexpr int kTileM = 320;
-constexpr int kTileN = 256;
-// K slices of 64 in a ring of two (copy of slice k + 1 in flight while slice
-// k is consumed).  Measured at M = 4800: slices of 32 in a ring of three or
-// four (prefetch distance 2-3) are 5% slower -- the loop is bound by LDS
-// traffic (copies plus operand reads, about 115 B/clock per CU), not by copy
-// latency.
-constexpr int kTileK = 64;
-constexpr int kStages = 2;
-constexpr int kWaves = 8;
-constexpr int kThreads = 64 * kWaves;
-constexpr int kWaveM = 160;                       // rows per wavefront
-constexpr int kWaveN = 64;                        // columns per wavefront
-constexpr int kBM = kWaveM / 32;                  // 5 row blocks
-constexpr int kBN = kWaveN / 32;                  // 2 column blocks
-constexpr int kRowBytes = kTileK * 2;             // bytes per LDS row
-constexpr int kChunks = kRowBytes / 16;           // 16-byte chunks per row
-constexpr int kRowsPerCopy = 1024 / kRowBytes;    // rows per 1 KB copy instruction
-constexpr int kStageA = kTileM * kRowBytes;
-constexpr int kStageB = kTileN * kRowBytes;
-constexpr int kStage = kStageA + kStageB;
-constexpr int kCopiesA = kStageA / 1024;
-constexpr int kCopies = kStage / 1024;            // copy instructions per slice
-constexpr int kCopySlots = (kCopies + kWaves - 1) / kWaves;
-constexpr int kFullWaves = kCopies - kWaves * (kCopySlots - 1);  // wavefronts issuing kCopySlots copies
-constexpr int kEpiWave = kWaveM * kWaveN * 2;     // 20 KB of fp16 per wavefront
-constexpr int kLdsBytes = kStages * kStage > kWaves * kEpiWave ? kStages * kStage : kWaves * kEpiWave;
-static_assert(kChunks == 4 || kChunks == 8, "32- or 64-wide K slices");
+typedef void (*KernelFn)(TileParams);
 
-// Chunk position of 16-byte chunk c of LDS row r: c ^ swz(r).  A 16-lane
-// group reads 16 consecutive rows at one logical chunk; the map spreads them
-// over all 64 banks (rows of 64 bytes: 4 per 64 banks; of 128: 2).
-__device__ __forceinline__ int row_swz(int r) { return kChunks == 8 ? (r >> 1) & 7 : (r >> 2) & 3; }
-static_assert(kLdsBytes <= 160 * 1024, "LDS budget of one CU");
-
-#define LDS_PTR(T, p) ((__attribute__((address_space(3))) T*)(p))
-
-struct GemmParams {
-  const _Float16* x;
-  const _Float16* w;
-  const _Float16* bias;
-  _Float16* y;
-  int ldx, ldw, ldy;  // row strides (elements)
-  int M, N, K;
-  int tiles_m;
-  int act;  // 1: SiLU
+struct TileKernel {
+  int bm, bn, threads;
+  KernelFn fn[4];  // by epilogue; null where that epilogue has no use for the shape
 };
 
-// Copy of 1 KB (8 rows of 128 bytes) global -> LDS; lane l's 16 bytes land
-// at lds_addr + 16 l.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void dma_1k(uint32_t lds_addr, const char* gbase, uint32_t voff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(lds_addr), "v"(voff), "s"(gbase) : "memory", "m0");
+#define SIDON_TILE(BM, BN, WM, WN, MF, ST, GLU, F32)                                       \
+  {BM, BN, 64 * WM * WN,                                                                   \
+   {gemm_tile_kernel<BM, BN, WM, WN, MF, ST, kHalf>, GLU(BM, BN, WM, WN, MF, ST, kGlu),    \
+    F32(BM, BN, WM, WN, MF, ST, kPart), F32(BM, BN, WM, WN, MF, ST, kAdd)}}
+#define SIDON_HAS(BM, BN, WM, WN, MF, ST, MODE) gemm_tile_kernel<BM, BN, WM, WN, MF, ST, MODE>
+#define SIDON_NOT(BM, BN, WM, WN, MF, ST, MODE) nullptr
+
+// The shapes that some measured (M, N, K) needs: a mean of 0.3% over the best
+// of 22 shapes.  One workgroup of the larger ones fills a CU's LDS.  256 wide
+// ones only where an fp16 output is wide enough to need them.
+const TileKernel kTiles[] = {
+    SIDON_TILE(32, 64, 2, 2, 16, 6, SIDON_HAS, SIDON_HAS),
+    SIDON_TILE(64, 64, 2, 2, 16, 4, SIDON_HAS, SIDON_HAS),
+    SIDON_TILE(96, 64, 2, 2, 16, 4, SIDON_HAS, SIDON_HAS),
+    SIDON_TILE(128, 64, 4, 2, 16, 4, SIDON_HAS, SIDON_HAS),
+    SIDON_TILE(160, 64, 2, 2, 16, 4, SIDON_HAS, SIDON_HAS),
+    SIDON_TILE(64, 128, 2, 4, 16, 4, SIDON_HAS, SIDON_HAS),
+    SIDON_TILE(96, 128, 2, 2, 16, 4, SIDON_HAS, SIDON_HAS),
+    SIDON_TILE(128, 128, 2, 4, 16, 4, SIDON_HAS, SIDON_HAS),
+    SIDON_TILE(160, 128, 2, 2, 16, 3, SIDON_HAS, SIDON_HAS),
+    SIDON_TILE(192, 128, 2, 4, 16, 3, SIDON_HAS, SIDON_HAS),
+    SIDON_TILE(128, 256, 2, 4, 16, 3, SIDON_HAS, SIDON_NOT),
+    SIDON_TILE(160, 256, 1, 4, 32, 3, SIDON_HAS, SIDON_NOT),
+    SIDON_TILE(192, 256, 2, 4, 16, 2, SIDON_NOT, SIDON_NOT),
+    SIDON_TILE(256, 256, 2, 4, 16, 2, SIDON_NOT, SIDON_NOT),
+    SIDON_TILE(320, 256, 2, 4, 32, 2, SIDON_NOT, SIDON_NOT),
+};
+
+constexpr int kMaxSplits = 8;        // what the norm sums in one pass
+constexpr int kGroupM = 8;           // row tiles walked together (level with 4, better from M = 1600 on)
+// The partial tiles of a split projection hold at most this many rows in
+// all (splits x M), so that a caller's workspace is bounded.
+constexpr int64_t kMaxPartRows = 8192;
+
+struct Choice {
+  const TileKernel* tile = nullptr;
+  int splits = 1;
+  double us = 0;
+};
+
+Choice choose(int M, int N, int K, int mode, int max_splits) {
+  const int cus = sidon::compute_units();
+  const int slices = K / 64;
+  Choice best;
+  for (const TileKernel& t : kTiles) {
+    if (t.fn[mode] == nullptr || N % t.bn != 0) continue;
+    const int64_t tiles = (int64_t)((M + t.bm - 1) / t.bm) * (N / t.bn);
+    const double mm = t.bm * t.bn / 4096.0, cp = (t.bm + t.bn) / 64.0;
+    for (int s = 1; s <= max_splits; ++s) {
+      // At least two slices per split, and the splits of one round of CUs.
+      if (s > 1 && (2 * s > slices || tiles * s > cus || (int64_t)s * M > kMaxPartRows)) break;
+      const double n = (double)tiles * s;
+      const double load = (double)((tiles * s + cus - 1) / cus);
+      const double nk = (double)slices / s;
+      double us = 3.0 + load * (0.062 * nk * mm + 0.031 * nk + (mode <= kGlu ? 0.39 : 0.48) * mm) +
+                  0.065 * (n / cus) * nk * cp;
+      if (s > 1) us += (s + 1.0) * M * N * 4.0 / 1.5e7;  // partial tiles read back, the stream written by the norm
+      if (best.tile == nullptr || us < best.us) best = Choice{&t, s, us};
+    }
+  }
+  return best;
 }
-#pragma clang diagnostic pop
 
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() { asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N) : "memory"); }
-
-// Wait until slice kt has landed while up to `newer` later slices (of kPer
-// copies each, issued after it by this wavefront) stay in flight.
-template <int kPer>
-__device__ __forceinline__ void wait_slice(int newer) {
-  if (newer >= 2) {
-    wait_vmcnt<2 * kPer>();
-  } else if (newer == 1) {
-    wait_vmcnt<kPer>();
-  } else {
-    wait_vmcnt<0>();
-  }
+// Operands as the kernel's 16-byte copies and 32-bit offsets need them.
+bool operands_fit(int64_t M, int64_t N, int ldx, int ldw, const void* x, const void* w) {
+  return ldx % 8 == 0 && ldw % 8 == 0 && M * ldx * 2 < (int64_t(1) << 32) && N * ldw * 2 < (int64_t(1) << 32) &&
+         sidon::aligned16(x) && sidon::aligned16(w);
 }
 
-// SiLU as the encoder's in-place SiLU kernel computes it (fp32, hardware
-// exponential and reciprocal, rounded to fp16); the empty asm keeps the
-// product and the conversion from fusing into one mixed-precision rounding.
-__device__ __forceinline__ _Float16 silu16(_Float16 h) {
-  const float x = (float)h;
-  float y = x * __builtin_amdgcn_rcpf(1.f + __expf(-x));
-  asm volatile("" : "+v"(y));
-  return (_Float16)y;
+int launch(const Choice& c, int mode, TileParams p, hipStream_t stream, const char* what) {
+  p.tiles_m = (p.M + c.tile->bm - 1) / c.tile->bm;
+  p.tiles_n = p.N / c.tile->bn;
+  p.splits = c.splits;
+  p.group = p.tiles_m < kGroupM ? p.tiles_m : kGroupM;
+  const int64_t wgs = (int64_t)p.tiles_m * p.tiles_n * p.splits;
+  if (wgs >= (int64_t(1) << 31)) return fail(SIDON_E_SHAPE, "too many tiles");
+  hipLaunchKernelGGL(c.tile->fn[mode], dim3((unsigned)wgs), dim3(c.tile->threads), 0, stream, p);
+  const hipError_t err = hipGetLastError();
+  if (err != hipSuccess) return fail(SIDON_E_LAUNCH, "%s launch failed: %s", what, hipGetErrorString(err));
+  return SIDON_OK;
 }
 
-__global__ void __launch_bounds__(kThreads) gemm_bias_act_kernel(const GemmParams p) {
-  __shared__ __attribute__((aligned(16))) char smem[kLdsBytes];
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wm = w >> 2;  // 0..1
-  const int wn = w & 3;   // 0..3
+TileParams params(const void* x, int ldx, const void* w, int ldw, const void* bias, void* y, int ldy, int M, int N,
+                  int K, int act) {
+  TileParams p{};
+  p.x = static_cast<const _Float16*>(x);
+  p.w = static_cast<const _Float16*>(w);
+  p.bias = static_cast<const _Float16*>(bias);
+  p.y = y;
+  p.ldx = ldx;
+  p.ldw = ldw;
+  p.ldy = ldy;
+  p.M = M;
+  p.N = N;
+  p.K = K;
+  p.act = act;
+  return p;
+}
 
-  // Tiles are numbered with M fastest; each XCD (workgroups are dispatched
-  // round-robin over the 8) takes a contiguous range, so its tiles share a
-  // few column blocks of W, which stay in its L2.
-  const int nwg = gridDim.x;
-  const int bid = blockIdx.x;
-  const int xcd = bid & 7;
-  const int per = nwg >> 3;
-  const int rem = nwg & 7;
-  const int lin = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + (bid >> 3);
-  const int tn = lin / p.tiles_m;
-  const int tm = lin - tn * p.tiles_m;
-  const int m0 = tm * kTileM;
-  const int n0 = tn * kTileN;
+bool res_fits(int M, int N, int K) { return M >= 1 && N >= 64 && N % 64 == 0 && K >= 128 && K % 128 == 0; }
 
-  // Copy instruction i (of kCopies per slice; wavefront w issues i = w + 8 j):
-  // rows kRowsPerCopy i' + lane / kChunks of the X slice (i < kCopiesA) or of
-  // the W slice; lane offsets fixed for the whole loop (X rows >= M re-read
-  // row M - 1, whose results are never stored).
-  const uint32_t lds0 = (uint32_t)(uintptr_t)LDS_PTR(char, smem);
-  uint32_t voff[kCopySlots];
-#pragma unroll
-  for (int j = 0; j < kCopySlots; ++j) {
-    const int i = min(w + kWaves * j, kCopies - 1);
-    const bool xi = i < kCopiesA;
-    const int r = (xi ? kRowsPerCopy * i : kRowsPerCopy * (i - kCopiesA)) + lane / kChunks;
-    const int c = (lane % kChunks) ^ row_swz(r);  // global chunk that lands at chunk position lane % kChunks
-    voff[j] = xi ? (uint32_t)min(m0 + r, p.M - 1) * (uint32_t)p.ldx * 2u + (uint32_t)c * 16u
-                 : (uint32_t)(n0 + r) * (uint32_t)p.ldw * 2u + (uint32_t)c * 16u;
-  }
-  const char* xg = reinterpret_cast<const char*>(p.x);
-  const char* wg = reinterpret_cast<const char*>(p.w);
-  auto issue = [&](int kt) {
-    const uint32_t base = lds0 + (kt % kStages) * kStage;
-#pragma unroll
-    for (int j = 0; j < kCopySlots; ++j) {
-      const int i = w + kWaves * j;
-      if (i < kCopies) {  // wave-uniform
-        const bool xi = i < kCopiesA;
-        dma_1k(base + i * 1024, (xi ? xg : wg) + kt * kRowBytes, voff[j]);
-      }
-    }
-  };
-
-  // Operand reads: lane (n, g) reads LDS row r = 32 blk + n, chunk 2 s + g
-  // (k = 16 s + 8 g + [0, 8) of the slice) for k16 step s.
-  const int ln = lane & 31;
-  const int lg = lane >> 5;
-  int aoff[kBM], boff[kBN];  // row byte offsets within a stage
-#pragma unroll
-  for (int b = 0; b < kBM; ++b) aoff[b] = (kWaveM * wm + 32 * b + ln) * kRowBytes;
-#pragma unroll
-  for (int b = 0; b < kBN; ++b) boff[b] = kStageA + (kWaveN * wn + 32 * b + ln) * kRowBytes;
-  const int swz = row_swz(ln);  // rows 32 b + ln share the swizzle of row ln
-
-  f32x16 acc[kBM][kBN];
-#pragma unroll
-  for (int i = 0; i < kBM; ++i)
-#pragma unroll
-    for (int j = 0; j < kBN; ++j) acc[i][j] = f32x16{};
-
-  const int kslices = p.K / kTileK;
-#pragma unroll
-  for (int kt = 0; kt < kStages - 1; ++kt)
-    if (kt < kslices) issue(kt);
-  for (int kt = 0; kt < kslices; ++kt) {
-    // Slice kt has landed for every wavefront, and nobody reads slice kt - 1
-    // any more, whose buffer the copy of slice kt + kStages - 1 refills.
-    const int newer = min(kStages - 2, kslices - 1 - kt);
-    if (w < kFullWaves) {
-      wait_slice<kCopySlots>(newer);
-    } else {
-      wait_slice<kCopySlots - 1>(newer);
-    }
-    __syncthreads();
-    if (kt + kStages - 1 < kslices) issue(kt + kStages - 1);
-    const char* st = smem + (kt % kStages) * kStage;
-    // Operands of k16 step s + 1 are read while the 10 MFMAs of step s run
-    // (two register sets; the scheduling barriers keep the compiler from
-    // interleaving the reads into the MFMA group, where each would wait).
-    h8 xa[2][kBM], wb[2][kBN];
-    auto load = [&](int s, int set) SIDON_INLINE {
-      const int chunk = ((2 * s + lg) ^ swz) << 4;
-#pragma unroll
-      for (int b = 0; b < kBM; ++b) xa[set][b] = *reinterpret_cast<const h8*>(st + aoff[b] + chunk);
-#pragma unroll
-      for (int b = 0; b < kBN; ++b) wb[set][b] = *reinterpret_cast<const h8*>(st + boff[b] + chunk);
-    };
-    load(0, 0);
-#pragma unroll
-    for (int s = 0; s < kTileK / 16; ++s) {
-      const int cur = s & 1;
-      if (s + 1 < kTileK / 16) load(s + 1, cur ^ 1);
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < kBM; ++i)
-#pragma unroll
-        for (int j = 0; j < kBN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wb[cur][j], xa[cur][i], acc[i][j], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  __syncthreads();  // every wavefront is done with the ring (the epilogue reuses it)
-
-  // Epilogue.  acc[i][j] is Y^T for rows 32 i + n (lane column n) and
-  // columns 32 j + 8 (e / 4) + 4 g + (e % 4): four consecutive columns per
-  // group e / 4.  Bias add (rounded to fp16 as addmm stores it), SiLU, and
-  // the fp16 tile of this wavefront into its own 20 KB of LDS (row stride
-  // 128 bytes, 8-byte unit u at u ^ (row & 15)), then whole rows out.
-  char* ep = smem + w * kEpiWave;
-#pragma unroll
-  for (int j = 0; j < kBN; ++j) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int col = kWaveN * wn + 32 * j + 8 * q + 4 * lg;  // within the tile
-      h4 bv = {};
-      if (p.bias != nullptr) bv = *reinterpret_cast<const h4*>(p.bias + n0 + col);
-#pragma unroll
-      for (int i = 0; i < kBM; ++i) {
-        h4 v;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          _Float16 hsum = (_Float16)(acc[i][j][4 * q + e] + (float)bv[e]);
-          v[e] = p.act == 1 ? silu16(hsum) : hsum;
-        }
-        const int row = 32 * i + ln;                 // within the wavefront's 160
-        const int unit = (col - kWaveN * wn) >> 2;   // 8-byte unit within the 128-byte row
-        *reinterpret_cast<h4*>(ep + row * 128 + ((unit ^ (row & 15)) << 3)) = v;
-      }
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): own LDS writes done (wave-private region)
-  // Rows 8 t + lane / 8, 16-byte chunk lane % 8 (units 2 c, 2 c + 1).
-  const int c = lane & 7;
-#pragma unroll 4
-  for (int t = 0; t < kWaveM / 8; ++t) {
-    const int row = 8 * t + (lane >> 3);
-    const int gm = m0 + kWaveM * wm + row;
-    const h4 lo = *reinterpret_cast<const h4*>(ep + row * 128 + (((2 * c) ^ (row & 15)) << 3));
-    const h4 hi = *reinterpret_cast<const h4*>(ep + row * 128 + (((2 * c + 1) ^ (row & 15)) << 3));
-    if (gm < p.M) {
-      const h8 v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-      *reinterpret_cast<h8*>(p.y + (int64_t)gm * p.ldy + n0 + kWaveN * wn + 8 * c) = v;
-    }
-  }
+// Whether the byte ranges of x [M, K] or w [N, K] and of y (rows of
+// `y_row` bytes, ldy_bytes apart) overlap: workgroups read X and W while
+// others already write Y.
+bool overlaps(const void* x, int ldx, const void* w, int ldw, const void* y, int64_t ldy_bytes, int64_t y_row, int M,
+              int N, int K) {
+  const uintptr_t xb = reinterpret_cast<uintptr_t>(x), wb = reinterpret_cast<uintptr_t>(w);
+  const uintptr_t yb = reinterpret_cast<uintptr_t>(y);
+  const uintptr_t xe = xb + (uintptr_t)(((int64_t)(M - 1) * ldx + K) * 2);
+  const uintptr_t we = wb + (uintptr_t)(((int64_t)(N - 1) * ldw + K) * 2);
+  const uintptr_t ye = yb + (uintptr_t)((int64_t)(M - 1) * ldy_bytes + y_row);
+  return (xb < ye && yb < xe) || (wb < ye && yb < we);
 }
 
 }  // namespace
 
-SIDON_API int sidon_gemm_bias_act_fits(int M, int N, int K) {
-  return M >= 1 && N >= kTileN && N % kTileN == 0 && K >= kTileK && K % kTileK == 0 ? 1 : 0;
+namespace sidon {
+
+// Up to here the kernel is faster than hipBLASLt at every measured shape;
+// past it the library's 256 x 256 kernels win (M x 3072 x 1024: M = 3000 23.9
+// against 30.8 us, 3600 30.5 against 27.6; M x 4096: 2000 23.0 against 24.1
+// without its SiLU, 3000 32.9 against 28.7).
+bool gemm_half_preferred(int M, int N, int K) {
+  return M >= 1 && N >= 64 && N % 64 == 0 && K >= 64 && K % 64 == 0 && (int64_t)M * N <= (int64_t)9 << 20;
 }
 
-// One workgroup per CU (its LDS fills one): the kernel pays off when its
-// tiles keep at least three quarters of the CUs busy in every dispatch round
-// (at N = 4096, K = 1024: M = 4800 gives 240 tiles on 256 CUs, 17% faster
-// than hipBLASLt's GEMM followed by the SiLU pass; M = 1500 gives 80 and is
-// slower).
+bool gemm_half_takes(const void* x, int ldx, const void* w, int ldw, const void* bias, const void* y, int ldy, int M,
+                     int N, int K) {
+  return gemm_half_preferred(M, N, K) && operands_fit(M, N, ldx, ldw, x, w) && ldy % 8 == 0 && aligned16(y) &&
+         (reinterpret_cast<uintptr_t>(bias) & 7u) == 0 &&
+         !overlaps(x, ldx, w, ldw, y, (int64_t)ldy * 2, (int64_t)N * 2, M, N, K);
+}
+
+int gemm_half(const void* x, int ldx, const void* w, int ldw, const void* bias, void* y, int ldy, int M, int N, int K,
+              int act, void* stream) {
+  return launch(choose(M, N, K, kHalf, 1), kHalf,
+                params(x, ldx, w, ldw, bias, y, ldy, M, N, K, act == 1 ? kSilu : kNone),
+                reinterpret_cast<hipStream_t>(stream), "gemm");
+}
+
+}  // namespace sidon
+
+SIDON_API int sidon_gemm_bias_act_fits(int M, int N, int K) {
+  return M >= 1 && N >= 256 && N % 256 == 0 && K >= 64 && K % 64 == 0 ? 1 : 0;
+}
+
+// Against the library with the SiLU in its epilogue this pays off past
+// gemm_half_preferred's range where 320 x 256 tiles, one per CU, keep four
+// fifths of the CUs busy in every round (M x 4096 x 1024: 4200 45.9 against
+// 56.7 us, 4800 47.0 against 47.0 without its SiLU; 3600, 192 tiles, 40 against 32.5).
 SIDON_API int sidon_gemm_bias_act_preferred(int M, int N, int K) {
   if (!sidon_gemm_bias_act_fits(M, N, K)) return 0;
   if (sidon::check_device() != SIDON_OK) return 0;
-  const int64_t tiles = (int64_t)((M + kTileM - 1) / kTileM) * (N / kTileN);
+  const int64_t tiles = (int64_t)((M + 319) / 320) * (N / 256);
   const int64_t cus = sidon::compute_units();
   const int64_t rounds = (tiles + cus - 1) / cus;
-  return 4 * tiles >= 3 * rounds * cus ? 1 : 0;
+  return !sidon::gemm_half_preferred(M, N, K) && 5 * tiles >= 4 * rounds * cus ? 1 : 0;
 }
 
 SIDON_API int sidon_gemm_bias_act(const void* x, int ldx, const void* w, int ldw, const void* bias, void* y, int ldy,
                                   int M, int N, int K, int act, sidon_stream_t stream) {
-  using sidon::fail;
   sidon::clear_error();
   if (!x || !w || !y) return fail(SIDON_E_NULL, "x, w and y must be non-NULL");
   if (!sidon_gemm_bias_act_fits(M, N, K))
-    return fail(SIDON_E_SHAPE, "M=%d N=%d K=%d: need M >= 1, N a multiple of %d, K a multiple of %d", M, N, K,
-                kTileN, kTileK);
+    return fail(SIDON_E_SHAPE, "M=%d N=%d K=%d: need M >= 1, N a multiple of 256, K a multiple of 64", M, N, K);
   if (ldx < K || ldw < K || ldy < N || (ldx | ldw | ldy) % 8 != 0)
     return fail(SIDON_E_STRIDE, "row strides ldx=%d ldw=%d ldy=%d must be multiples of 8 and >= K, K, N", ldx, ldw,
                 ldy);
@@ -314,24 +225,95 @@ SIDON_API int sidon_gemm_bias_act(const void* x, int ldx, const void* w, int ldw
     return fail(SIDON_E_ALIGN, "x, w, y must be 16-byte aligned and bias 8-byte aligned");
   int rc;
   if ((rc = sidon::check_device())) return rc;
-  GemmParams p;
-  p.x = static_cast<const _Float16*>(x);
-  p.w = static_cast<const _Float16*>(w);
-  p.bias = static_cast<const _Float16*>(bias);
-  p.y = static_cast<_Float16*>(y);
-  p.ldx = ldx;
-  p.ldw = ldw;
-  p.ldy = ldy;
-  p.M = M;
-  p.N = N;
-  p.K = K;
-  p.tiles_m = (M + kTileM - 1) / kTileM;
-  p.act = act;
-  const int64_t tiles = (int64_t)p.tiles_m * (N / kTileN);
-  if (tiles >= (int64_t(1) << 31)) return fail(SIDON_E_SHAPE, "too many tiles");
-  hipLaunchKernelGGL(gemm_bias_act_kernel, dim3((unsigned)tiles), dim3(kThreads), 0,
-                     reinterpret_cast<hipStream_t>(stream), p);
-  const hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return fail(SIDON_E_LAUNCH, "gemm launch failed: %s", hipGetErrorString(err));
-  return SIDON_OK;
+  return launch(choose(M, N, K, kHalf, 1), kHalf,
+                params(x, ldx, w, ldw, bias, y, ldy, M, N, K, act == 1 ? kSiluHalf : kNone),
+                reinterpret_cast<hipStream_t>(stream), "gemm");
+}
+
+SIDON_API int sidon_gemm_half_preferred(int M, int N, int K) {
+  if (!sidon::gemm_half_preferred(M, N, K)) return 0;
+  return sidon::check_device() == SIDON_OK ? 1 : 0;
+}
+
+SIDON_API int sidon_gemm_glu(const void* x, int ldx, const void* w, int ldw, void* y, int ldy, int M, int C, int K,
+                             sidon_stream_t stream) {
+  sidon::clear_error();
+  if (!x || !w || !y) return fail(SIDON_E_NULL, "x, w and y must be non-NULL");
+  if (M < 1 || C < 32 || C % 32 != 0 || C > (1 << 29) || K < 64 || K % 64 != 0)
+    return fail(SIDON_E_SHAPE, "M=%d C=%d K=%d: need M >= 1, C a multiple of 32, K a multiple of 64", M, C, K);
+  if (ldx < K || ldw < K || ldy < C || (ldx | ldw | ldy) % 8 != 0)
+    return fail(SIDON_E_STRIDE, "row strides ldx=%d ldw=%d ldy=%d must be multiples of 8 and >= K, K, C", ldx, ldw,
+                ldy);
+  if (!sidon::aligned16(x) || !sidon::aligned16(w) || !sidon::aligned16(y))
+    return fail(SIDON_E_ALIGN, "x, w and y must be 16-byte aligned");
+  const int N = 2 * C;
+  if (!operands_fit(M, N, ldx, ldw, x, w)) return fail(SIDON_E_SHAPE, "X and W must each span less than 4 GiB");
+  if (overlaps(x, ldx, w, ldw, y, (int64_t)ldy * 2, (int64_t)C * 2, M, N, K))
+    return fail(SIDON_E_SHAPE, "x and w must not overlap y");
+  int rc;
+  if ((rc = sidon::check_device())) return rc;
+  return launch(choose(M, N, K, kGlu, 1), kGlu, params(x, ldx, w, ldw, nullptr, y, ldy, M, N, K, 0),
+                reinterpret_cast<hipStream_t>(stream), "gemm + GLU");
+}
+
+SIDON_API int sidon_gemm_res_fits(int M, int N, int K) { return res_fits(M, N, K) ? 1 : 0; }
+
+// The library's kernels were slower at every measured M of the encoder's two
+// residual shapes (25-4800, N = 1024); past the measured range they are kept.
+SIDON_API int sidon_gemm_res_preferred(int M, int N, int K) {
+  if (!res_fits(M, N, K) || (int64_t)M * N > (int64_t)5 << 20) return 0;
+  return sidon::check_device() == SIDON_OK ? 1 : 0;
+}
+
+SIDON_API int sidon_gemm_res(const void* x, int ldx, const void* w, int ldw, float* y, int ldy, int M, int N, int K,
+                             sidon_stream_t stream) {
+  sidon::clear_error();
+  if (!x || !w || !y) return fail(SIDON_E_NULL, "x, w and y must be non-NULL");
+  if (!res_fits(M, N, K))
+    return fail(SIDON_E_SHAPE, "M=%d N=%d K=%d: need M >= 1, N a multiple of 64, K a multiple of 128", M, N, K);
+  if (ldx < K || ldw < K || ldy < N || ldx % 8 != 0 || ldw % 8 != 0 || ldy % 4 != 0)
+    return fail(SIDON_E_STRIDE, "row strides ldx=%d ldw=%d (multiples of 8, >= K) ldy=%d (multiple of 4, >= N)", ldx,
+                ldw, ldy);
+  if ((int64_t)M * ldx * 2 >= (int64_t(1) << 32) || (int64_t)N * ldw * 2 >= (int64_t(1) << 32))
+    return fail(SIDON_E_SHAPE, "X and W must each span less than 4 GiB");
+  if (!sidon::aligned16(x) || !sidon::aligned16(w) || !sidon::aligned16(y))
+    return fail(SIDON_E_ALIGN, "x, w and y must be 16-byte aligned");
+  if (overlaps(x, ldx, w, ldw, y, (int64_t)ldy * 4, (int64_t)N * 4, M, N, K))
+    return fail(SIDON_E_SHAPE, "x and w must not overlap y (the kernel reads them while adding into y)");
+  int rc;
+  if ((rc = sidon::check_device())) return rc;
+  return launch(choose(M, N, K, kAdd, 1), kAdd, params(x, ldx, w, ldw, nullptr, y, ldy, M, N, K, 0),
+                reinterpret_cast<hipStream_t>(stream), "residual gemm");
+}
+
+SIDON_API int sidon_gemm_part_splits(int M, int N, int K) {
+  if (!res_fits(M, N, K) || sidon::check_device() != SIDON_OK) return 0;
+  return choose(M, N, K, kPart, kMaxSplits).splits;
+}
+
+SIDON_API int64_t sidon_gemm_part_rows(int M) { return M > kMaxPartRows ? M : kMaxPartRows; }
+
+SIDON_API int sidon_gemm_part(const void* x, int ldx, const void* w, int ldw, float* part, int64_t part_elems, int M,
+                              int N, int K, sidon_stream_t stream) {
+  sidon::clear_error();
+  if (!x || !w || !part) return fail(SIDON_E_NULL, "x, w and part must be non-NULL");
+  if (!res_fits(M, N, K))
+    return fail(SIDON_E_SHAPE, "M=%d N=%d K=%d: need M >= 1, N a multiple of 64, K a multiple of 128", M, N, K);
+  if (ldx < K || ldw < K || ldx % 8 != 0 || ldw % 8 != 0)
+    return fail(SIDON_E_STRIDE, "row strides ldx=%d ldw=%d must be multiples of 8 and >= K", ldx, ldw);
+  if (!sidon::aligned16(x) || !sidon::aligned16(w) || !sidon::aligned16(part))
+    return fail(SIDON_E_ALIGN, "x, w and part must be 16-byte aligned");
+  if (!operands_fit(M, N, ldx, ldw, x, w)) return fail(SIDON_E_SHAPE, "X and W must each span less than 4 GiB");
+  int rc;
+  if ((rc = sidon::check_device())) return rc;
+  const Choice c = choose(M, N, K, kPart, kMaxSplits);
+  if (part_elems < (int64_t)c.splits * M * N)
+    return fail(SIDON_E_SHAPE, "part holds %lld values, %d splits of %d x %d need more", (long long)part_elems,
+                c.splits, M, N);
+  // The splits' tiles lie one after another: `splits` times M rows of N.
+  if (overlaps(x, ldx, w, ldw, part, (int64_t)N * 4, (int64_t)N * 4 + (int64_t)(c.splits - 1) * M * N * 4, M, N, K))
+    return fail(SIDON_E_SHAPE, "x and w must not overlap part");
+  TileParams p = params(x, ldx, w, ldw, nullptr, part, N, M, N, K, 0);
+  p.split_stride = (int64_t)M * N;
+  return launch(c, kPart, p, reinterpret_cast<hipStream_t>(stream), "partial gemm");
 }

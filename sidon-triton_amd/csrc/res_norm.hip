@@ -137,6 +137,127 @@ __global__ void __launch_bounds__(64 * kRowsPerBlock) res_norm_kernel(const RNPa
   }
 }
 
+// The norm behind a split residual projection: x += sum of the partial tiles,
+// and the norm of the sum (sidon_res_norm_parts).  One row per block of four
+// wavefronts (chunk j of wavefront u's lane l: columns 4 (64 (4 j + u) + l)),
+// so that a short chunk's rows spread over the chip; every load of a row -- x,
+// its partial tiles, bias, norm weights -- is in flight before the first sum.
+// Bound by that one memory round trip: with C = 1024, 2 to 8 splits take 2.8
+// to 3.0 us per launch at R = 150 (res_norm without the sums 2.3) and 4.4 to
+// 4.9 us at R = 750 (3.1); one wavefront per row took 4.3 and 5.5-6.4 us, two
+// 3.4 and 4.8-5.6.
+constexpr int kPartWaves = 4;
+
+struct PartParams {
+  float* x;
+  const float* part;
+  const float* bias;
+  const float* n1_w;
+  const float* n1_b;
+  const float* n2_w;
+  const float* n2_b;
+  _Float16* xn;
+  float eps1, eps2;
+  int splits, R, C;
+};
+
+constexpr int kMaxSplits = 8;
+
+template <int NC, bool kHasNorm1, bool kHasNorm2>
+__global__ void __launch_bounds__(64 * kPartWaves) res_norm_parts_kernel(const PartParams p) {
+  __shared__ float red[2][kPartWaves];
+  const int lane = threadIdx.x & 63;
+  const int u = threadIdx.x >> 6;
+  const int64_t base = (int64_t)blockIdx.x * p.C;
+  const int64_t stride = (int64_t)p.R * p.C;
+  f4 v[NC], t[NC][kMaxSplits], bv[NC], w1[NC], b1[NC], w2[NC], b2[NC];
+  auto col = [&](int j) { return 4 * (64 * (kPartWaves * j + u) + lane); };
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    const int c = col(j);
+    const bool in = c < p.C;
+    const f4 zero = {0.f, 0.f, 0.f, 0.f};
+    v[j] = in ? *reinterpret_cast<const f4*>(p.x + base + c) : zero;
+#pragma unroll
+    for (int s = 0; s < kMaxSplits; ++s)
+      t[j][s] = in && s < p.splits ? *reinterpret_cast<const f4*>(p.part + s * stride + base + c) : zero;
+    bv[j] = in && p.bias != nullptr ? *reinterpret_cast<const f4*>(p.bias + c) : zero;
+    if constexpr (kHasNorm1) {
+      w1[j] = in ? *reinterpret_cast<const f4*>(p.n1_w + c) : zero;
+      b1[j] = in ? *reinterpret_cast<const f4*>(p.n1_b + c) : zero;
+    }
+    if constexpr (kHasNorm2) {
+      w2[j] = in ? *reinterpret_cast<const f4*>(p.n2_w + c) : zero;
+      b2[j] = in ? *reinterpret_cast<const f4*>(p.n2_b + c) : zero;
+    }
+  }
+  // Sum over the row; `which` alternates the LDS words of successive calls.
+  auto row_sum = [&](float s, int which) {
+    s = wave_sum(s);
+    if (lane == 0) red[which][u] = s;
+    __syncthreads();
+    return (red[which][0] + red[which][1]) + (red[which][2] + red[which][3]);
+  };
+  auto norm = [&](const f4(&w)[NC], const f4(&b)[NC], float eps) {
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) s += (v[j][0] + v[j][1]) + (v[j][2] + v[j][3]);
+    const float mean = row_sum(s, 0) / (float)p.C;
+    float q = 0.f;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+      if (col(j) < p.C) {
+        v[j] -= mean;
+        q += (v[j][0] * v[j][0] + v[j][1] * v[j][1]) + (v[j][2] * v[j][2] + v[j][3] * v[j][3]);
+      }
+    }
+    const float rstd = rsqrtf(row_sum(q, 1) / (float)p.C + eps);
+#pragma unroll
+    for (int j = 0; j < NC; ++j) v[j] = v[j] * rstd * w[j] + b[j];
+  };
+  auto store_x = [&]() {
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+      if (col(j) < p.C) *reinterpret_cast<f4*>(p.x + base + col(j)) = v[j];
+  };
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    f4 sum = t[j][0];
+#pragma unroll
+    for (int s = 1; s < kMaxSplits; ++s)
+      if (s < p.splits) sum += t[j][s];
+    v[j] += sum;
+  }
+  if constexpr (!kHasNorm1) store_x();
+#pragma unroll
+  for (int j = 0; j < NC; ++j) v[j] += bv[j];
+  if constexpr (kHasNorm1) {
+    norm(w1, b1, p.eps1);
+    store_x();
+  }
+  if constexpr (kHasNorm2) {
+    norm(w2, b2, p.eps2);
+#pragma unroll
+    for (int j = 0; j < NC; ++j)
+      if (col(j) < p.C) *reinterpret_cast<h4*>(p.xn + base + col(j)) = __builtin_convertvector(v[j], h4);
+  }
+}
+
+template <int NC>
+hipError_t launch_parts(const PartParams& p, hipStream_t stream) {
+  const dim3 grid(p.R), block(64 * kPartWaves);
+  if (p.n1_w && p.n2_w) {
+    hipLaunchKernelGGL((res_norm_parts_kernel<NC, true, true>), grid, block, 0, stream, p);
+  } else if (p.n1_w) {
+    hipLaunchKernelGGL((res_norm_parts_kernel<NC, true, false>), grid, block, 0, stream, p);
+  } else if (p.n2_w) {
+    hipLaunchKernelGGL((res_norm_parts_kernel<NC, false, true>), grid, block, 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((res_norm_parts_kernel<NC, false, false>), grid, block, 0, stream, p);
+  }
+  return hipGetLastError();
+}
+
 template <int NC>
 hipError_t launch(const RNParams& p, hipStream_t stream) {
   const int blocks = (p.R + kRowsPerBlock - 1) / kRowsPerBlock;
@@ -190,5 +311,31 @@ SIDON_API int sidon_res_norm(float* x, const float* y, const float* bias, const 
     default: err = launch<8>(p, s); break;
   }
   if (err != hipSuccess) return fail(SIDON_E_LAUNCH, "res_norm launch failed: %s", hipGetErrorString(err));
+  return SIDON_OK;
+}
+
+SIDON_API int sidon_res_norm_parts(float* x, const float* part, int splits, const float* bias, const float* n1_w,
+                                   const float* n1_b, float eps1, const float* n2_w, const float* n2_b, float eps2,
+                                   void* xn, int R, int C, sidon_stream_t stream) {
+  using sidon::aligned16;
+  using sidon::fail;
+  sidon::clear_error();
+  if (!x || !part) return fail(SIDON_E_NULL, "x and part must be non-NULL");
+  if ((n1_w == nullptr) != (n1_b == nullptr)) return fail(SIDON_E_NULL, "norm1 needs both weight and bias");
+  if ((n2_w == nullptr) != (n2_b == nullptr)) return fail(SIDON_E_NULL, "norm2 needs both weight and bias");
+  if (n2_w && !xn) return fail(SIDON_E_NULL, "norm2 needs an xn output");
+  if (R < 1 || C < 4 || C > 64 * 4 * kMaxChunks || (C & 3) != 0 || splits < 1 || splits > kMaxSplits)
+    return fail(SIDON_E_SHAPE, "R=%d must be >= 1, C=%d a multiple of 4 in [4, %d] and splits=%d in [1, %d]", R, C,
+                64 * 4 * kMaxChunks, splits, kMaxSplits);
+  const void* ptrs[] = {x, part, bias, n1_w, n1_b, n2_w, n2_b};
+  for (const void* ptr : ptrs)
+    if (ptr && !aligned16(ptr)) return fail(SIDON_E_ALIGN, "fp32 tensors must be 16-byte aligned");
+  if (xn && (reinterpret_cast<uintptr_t>(xn) & 7u) != 0) return fail(SIDON_E_ALIGN, "xn must be 8-byte aligned");
+  int rc;
+  if ((rc = sidon::check_device())) return rc;
+  const PartParams p{x, part, bias, n1_w, n1_b, n2_w, n2_b, static_cast<_Float16*>(xn), eps1, eps2, splits, R, C};
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const hipError_t err = C <= 256 * kPartWaves ? launch_parts<1>(p, s) : launch_parts<2>(p, s);
+  if (err != hipSuccess) return fail(SIDON_E_LAUNCH, "res_norm_parts launch failed: %s", hipGetErrorString(err));
   return SIDON_OK;
 }

@@ -16,15 +16,13 @@ Mirrors src/sidon_triton/triton_encoder.py:
     ``load_encoder`` also reads the reference's own ``encoder_triton.pt``
     (with ``torch.load(weights_only=True)``).
 
-Per layer the work is: res_norm (HIP), the QKV GEMM on hipBLASLt through
-torch, the residual projections into the fp32 stream (one HIP kernel while
-its 64 x 64 tiles fit one per CU, else hipBLASLt), the pointwise conv's first
-GEMM on rocBLAS with the kernel chosen by timing (``blas.gemm_nt``), the
-feed-forward input projections with bias and SiLU (one HIP GEMM kernel where
-its tiles fill the chip, else hipBLASLt with the bias and SiLU in its epilogue),
-the relative_key attention (HIP), and the conv module's GLU + causal
-depthwise conv + LayerNorm + SiLU as one HIP kernel reading the pointwise
-conv's output.  Every op launches on the current stream, reads no
+Per layer the work is: res_norm (HIP); the projections, on this library's tiled
+GEMM kernel (csrc/gemm.hip) with the bias, the SiLU or the GLU in its epilogue,
+the residual ones with K split over workgroups at short chunks and their partial
+sums added by the next norm; hipBLASLt (``conformer.linear``,
+``conformer.linear_silu_lt``) for the widest outputs, where it is faster;
+the relative_key attention (HIP), and the conv module's causal
+depthwise conv + LayerNorm + SiLU as one HIP kernel on the GLU's output.  Every op launches on the current stream, reads no
 device data on the host and, given a ``workspace``, allocates nothing, so a
 whole encoder call can be captured into one HIP graph per length bucket.
 """
@@ -37,10 +35,11 @@ from pathlib import Path
 import torch
 
 from .blas import gemm_nt
-from .conformer import (glu_causal_dw_norm, linear_silu, linear_silu_lt, linear_silu_preferred, residual_gemm,
-                        residual_gemm_preferred, silu_)
+from .conformer import (causal_dw_norm, glu_causal_dw_norm, linear, linear_glu, linear_glu_fits, linear_silu,
+                        linear_silu_lt, linear_silu_preferred, partial_values, residual_gemm, residual_partials,
+                        residual_splits, silu_)
 from .encoder_attention import flexrel_attention
-from .encoder_block import res_norm
+from .encoder_block import res_norm, res_norm_parts
 from .flexrel import HEAD_DIM, LEFT, NUM_POS, RIGHT
 
 ENCODER_FILE = "encoder_mi355x.safetensors"
@@ -184,13 +183,15 @@ class HipEncoder:
     def workspace(self, rows: int) -> dict:
         """Buffers for calls of up to ``rows`` = B*L rows (graph capture
         reuses them): normalized features, the normed stream, one fp16 buffer
-        for the FFN intermediate / fused QKV / pointwise conv output (their
-        lifetimes do not overlap), and the attention context / conv output."""
+        for the FFN intermediate / fused QKV / GLU output (their lifetimes do
+        not overlap), the attention context / conv output, and the partial
+        sums of the residual projections of short chunks."""
         wide = max(self.inter, 3 * self.hidden)
         f16 = dict(device=self.device, dtype=torch.float16)
         return {"rows": rows, "fn": torch.empty(rows * self.features, device=self.device),
                 "xn": torch.empty(rows * self.hidden, **f16), "wide": torch.empty(rows * wide, **f16),
-                "ctx": torch.empty(rows * self.hidden, **f16)}
+                "ctx": torch.empty(rows * self.hidden, **f16),
+                "part": torch.empty(partial_values(rows, self.hidden), device=self.device)}
 
     @torch.no_grad()
     def __call__(self, features: torch.Tensor, frames: torch.Tensor | None = None,
@@ -218,7 +219,7 @@ class HipEncoder:
         ctx = ws["ctx"][:rows * hid].view(rows, hid)
         h_buf = wide[:rows * self.inter].view(rows, self.inter)
         qkv_buf = wide[:rows * 3 * hid].view(rows, 3 * hid)
-        pw1_buf = wide[:rows * 2 * hid].view(rows, 2 * hid)
+        part_buf = ws.get("part")
 
         feats = features.reshape(rows, nfeat)
         if feats.dtype != torch.float32 or not feats.is_contiguous():
@@ -240,30 +241,45 @@ class HipEncoder:
                 return linear_silu(xn, w, b, out=h_buf)
             return silu_(torch.addmm(b, xn, w.t(), out=h_buf))
 
-        own = {k: (residual_gemm_preferred(rows, hid, k, device) if self.own_residual is None
-                   else self.own_residual) for k in (hid, self.inter)}
+        # The residual projections: K split over workgroups with the partial
+        # sums added by the next norm (2+), in place on this library's kernel
+        # (1), or torch.addmm (0).
+        if self.own_residual is None:
+            split = {k: residual_splits(rows, hid, k, device) for k in (hid, self.inter)}
+            if part_buf is None:
+                split = {k: min(n, 1) for k, n in split.items()}
+        else:
+            split = dict.fromkeys((hid, self.inter), int(self.own_residual))
 
-        def res(a, w, bias, **kw):
-            # The residual projections: this library's kernel while its 64 x 64
-            # tiles fit one per CU (short chunks), else torch.addmm (hipBLASLt);
-            # rocBLAS's timed choice was no faster inside the encoder graph.
-            if own[a.shape[1]]:
+        def res(a, w, bias, norm1=None, norm2=None):
+            to = xn_buf if norm2 is not None else None
+            n = split[a.shape[1]]
+            if n > 1:
+                return res_norm_parts(x, residual_partials(a, w, part_buf), bias=bias, norm1=norm1, norm2=norm2, xn=to)
+            if n == 1:
                 residual_gemm(x, a, w)
             else:
                 torch.addmm(x, a, w.t(), out_dtype=torch.float32, out=x)
-            return res_norm(x, bias=bias, xn=xn_buf if kw.get("norm2") is not None else None, **kw)
+            return res_norm(x, bias=bias, norm1=norm1, write_x=norm1 is not None, norm2=norm2, xn=to)
+
+        def conv_in(p):
+            # GLU(xn . w^T), then the depthwise conv and its norm
+            if linear_glu_fits(xn, p["pw1_w"]):
+                g = linear_glu(xn, p["pw1_w"], out=wide[:rows * hid].view(rows, hid))
+                return causal_dw_norm(g, batch, p["dwt"], *p["dw_ln"], out=ctx)
+            pw1 = gemm_nt(xn, p["pw1_w"], wide[:rows * 2 * hid].view(rows, 2 * hid))
+            return glu_causal_dw_norm(pw1, batch, p["dwt"], *p["dw_ln"], out=ctx)
 
         for i, p in enumerate(layers):
             b1, b2, b4 = p["cum_bias"]
             last = i + 1 == len(layers)
             h = ffn_in(p["ffn1_w1"], p["ffn1_b1"])
-            xn = res(h, p["ffn1_w2"], b1, norm2=p["attn_ln"], write_x=False)
-            qkv = torch.addmm(p["qkv_b"], xn, p["qkv_w"].t(), out=qkv_buf)
+            xn = res(h, p["ffn1_w2"], b1, norm2=p["attn_ln"])
+            qkv = linear(xn, p["qkv_w"], p["qkv_b"], qkv_buf)
             c = flexrel_attention(qkv, batch, self.heads, p["rel"], lens, out=ctx)
-            xn = res(c, p["out_w"], b2, norm2=p["conv_ln"], write_x=False)
-            pw1 = gemm_nt(xn, p["pw1_w"], pw1_buf)
-            s = glu_causal_dw_norm(pw1, batch, p["dwt"], *p["dw_ln"], out=ctx)
-            xn = res(s, p["pw2_w"], b2, norm2=p["ffn2_ln"], write_x=False)
+            xn = res(c, p["out_w"], b2, norm2=p["conv_ln"])
+            s = conv_in(p)
+            xn = res(s, p["pw2_w"], b2, norm2=p["ffn2_ln"])
             h = ffn_in(p["ffn2_w1"], p["ffn2_b1"])
             xn = res(h, p["ffn2_w2"], b4, norm1=p["final_ln"],
                      norm2=None if last else layers[i + 1]["ffn1_ln"])

@@ -1,0 +1,158 @@
+"""The tiled GEMM kernel (csrc/gemm_tile.h) through each of its epilogues, at
+sizes that reach every tile shape the rule of csrc/gemm.hip picks on 256 compute
+units, one row past and before tile edges, and at fewer K slices than ring
+buffers; and the norm that adds a split projection's partial sums (needs an
+MI355X)."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = torch.device("cuda:0")
+
+
+def _operands(m, n, k, seed):
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    x = torch.randn(m, k, generator=gen, device=DEV).half()
+    w = (torch.randn(n, k, generator=gen, device=DEV) / k ** 0.5).half()
+    return x, w, gen
+
+
+def _sums(x, w):
+    """The float64 products, and a bound on the error of fp32 sums in any order."""
+    exact = x.double() @ w.double().t()
+    return exact, x.shape[1] * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 64, 64), (31, 128, 64), (33, 64, 128), (65, 192, 192), (97, 4096, 256), (129, 4096, 320), (333, 4096, 128),
+    (400, 4096, 1024), (500, 3072, 1024), (577, 3072, 1024), (577, 4096, 1024), (750, 3072, 1024), (751, 4096, 1024),
+    (1000, 4096, 192), (1463, 3072, 1024), (1601, 3072, 1024), (2000, 4096, 128), (2303, 4096, 1024),
+    (3000, 3072, 192), (9000, 1024, 64)])
+def test_linear_matches_float64(sidon, m, n, k):
+    """Bias, SiLU of the fp32 sum, one rounding: within half an fp16 step of the
+    float64 value plus the fp32 sums' own bound (the SiLU's slope is below
+    1.1); columns beside a strided output stay untouched."""
+    assert sidon._lib.load().sidon_gemm_half_preferred(m, n, k)
+    x, w, gen = _operands(m, n, k, m + n + k)
+    b = (torch.randn(n, generator=gen, device=DEV) * 0.1).half()
+    exact, bound = _sums(x, w)
+    exact = exact + b.double()
+    for act in (False, True):
+        wide = torch.full((m + 1, n + 16), 7.0, dtype=torch.float16, device=DEV)
+        out = sidon.conformer.linear_silu_lt(x, w, b, out=wide[:m, 8:n + 8], act=act)
+        want = torch.nn.functional.silu(exact) if act else exact
+        tol = 2.0 ** -11 * want.abs() + 1.1 * bound + 2.0 ** -20 * want.abs() + 2.0 ** -24
+        assert ((out.double() - want).abs() <= tol).all(), (act, float(((out.double() - want).abs() - tol).max()))
+        assert (wide[:, :8] == 7).all() and (wide[:, n + 8:] == 7).all() and (wide[m] == 7).all()
+
+
+@pytest.mark.parametrize("m,k", [(1, 64), (33, 128), (300, 1024), (650, 1024), (900, 192), (1000, 1024), (1463, 256),
+                                 (1601, 1024), (2500, 128), (3000, 1024), (3600, 192), (4200, 1024)])
+def test_linear_glu_is_the_projection_then_the_glu(sidon, m, k):
+    """Bit for bit what the projection followed by the GLU kernel gives: the
+    same sums in the same order, the same roundings."""
+    x, w, _ = _operands(m, 2048, k, m + k)
+    h = torch.empty(m, 2048, dtype=torch.float16, device=DEV)
+    want = sidon.conformer.glu(sidon.conformer.linear_silu(x, w, None, out=h, act=False))
+    assert torch.equal(sidon.conformer.linear_glu(x, w), want)
+
+
+def test_linear_glu_narrow_and_strided(sidon):
+    x, w, _ = _operands(70, 192, 192, 3)          # C = 96, one wavefront's columns past a power of two
+    wide = torch.full((70, 112), 7.0, dtype=torch.float16, device=DEV)
+    got = sidon.conformer.linear_glu(x, w, out=wide[:, 8:104])
+    h = (x.double() @ w.double().t()).half().double()
+    want = h[:, :96] * torch.sigmoid(h[:, 96:])
+    assert ((got.double() - want).abs() <= 2.0 ** -9 * want.abs() + 2.0 ** -12).all()
+    assert (wide[:, :8] == 7).all() and (wide[:, 104:] == 7).all()
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 64, 128), (33, 1024, 4096), (97, 1024, 4096), (150, 1024, 4096),
+                                   (200, 1024, 4096), (300, 1024, 4096), (577, 1024, 4096), (751, 1024, 4096),
+                                   (1463, 1024, 4096), (150, 1024, 1024), (400, 1024, 1024), (2500, 1024, 4096)])
+def test_partials_add_up_and_join_the_stream(sidon, m, n, k):
+    """The partial tiles' sum against float64, twice with the same bits; a
+    buffer of ``partial_values`` holds them; the norm adds them to the stream."""
+    x, w, gen = _operands(m, n, k, m + n + k)
+    exact, bound = _sums(x, w)
+    part = torch.full((sidon.conformer.partial_values(m, n),), float("nan"), device=DEV)
+    got = sidon.conformer.residual_partials(x, w, part)
+    assert got.shape[0] == sidon.conformer.residual_splits(m, n, k, DEV) and got.shape[0] >= 1
+    assert ((got.double().sum(0) - exact).abs() <= bound + 1e-12).all()
+    again = sidon.conformer.residual_partials(x, w, torch.empty_like(part))
+    assert torch.equal(again, got)
+    stream = torch.randn(m, n, generator=gen, device=DEV)
+    want = stream.double() + exact
+    sidon.encoder_block.res_norm_parts(stream, got)
+    # the sum of up to 9 fp32 terms: each addition rounds values below the bound
+    scale = got.double().abs().sum(0) + want.abs()
+    assert ((stream.double() - want).abs() <= bound + 9 * 2.0 ** -24 * scale).all()
+
+
+@pytest.mark.parametrize("rows,cols,splits", [(1, 4, 1), (3, 100, 2), (5, 1024, 8), (2, 1028, 3), (7, 2048, 5)])
+@pytest.mark.parametrize("first", [False, True])
+def test_res_norm_parts_matches_float64(sidon, rows, cols, splits, first):
+    gen = torch.Generator(device=DEV).manual_seed(rows + cols)
+
+    def r(*shape):
+        return torch.randn(*shape, generator=gen, device=DEV)
+
+    x, part, bias = r(rows, cols), r(splits, rows, cols), r(cols)
+    norms = [(1 + 0.1 * r(cols), 0.1 * r(cols), 1e-5) for _ in range(2)]
+    summed = x.double() + part.double().sum(0)
+
+    def ln(v, p):
+        return torch.nn.functional.layer_norm(v, (cols,), p[0].double(), p[1].double(), p[2])
+
+    stored = ln(summed + bias.double(), norms[0]) if first else summed
+    normed = ln(stored if first else summed + bias.double(), norms[1])
+    got = x.clone()
+    xn = sidon.encoder_block.res_norm_parts(got, part, bias=bias, norm1=norms[0] if first else None, norm2=norms[1])
+    # fp32 arithmetic on values of a few units; the fp16 output rounds once more
+    assert ((got.double() - stored).abs() <= 2e-5 * (1 + stored.abs())).all()
+    assert ((xn.double() - normed).abs() <= 2.0 ** -11 * normed.abs() + 4e-5).all()
+
+
+def test_split_projections_replay_like_eager(sidon):
+    """A captured projection, partial sums and norm, replayed three times with
+    eager work between, equal the eager calls."""
+    x, w, gen = _operands(150, 1024, 4096, 5)
+    ln = (torch.ones(1024, device=DEV), torch.zeros(1024, device=DEV), 1e-5)
+    start = torch.randn(150, 1024, generator=gen, device=DEV)
+    part = torch.empty(sidon.conformer.partial_values(150, 1024), device=DEV)
+    stream, xn = start.clone(), torch.empty(150, 1024, dtype=torch.float16, device=DEV)
+
+    def step():
+        sidon.encoder_block.res_norm_parts(stream, sidon.conformer.residual_partials(x, w, part), norm2=ln, xn=xn)
+
+    step()
+    want, want_n = stream.clone(), xn.clone()
+    graphs = sidon.graphs.BucketGraphs()
+    graphs.capture("step", step)
+    for rep in range(3):
+        stream.copy_(start)
+        xn.zero_()
+        part.zero_()
+        graphs.run("step", step)
+        torch.cuda.synchronize()
+        assert torch.equal(stream, want) and torch.equal(xn, want_n), rep
+        _ = (start * 2).sum().item()
+
+
+def test_residual_gemm_takes_the_split_or_the_strided_stream(sidon):
+    """K = 4096 into a contiguous stream (split) and into a strided one (in
+    place): the same sums up to their order."""
+    x, w, gen = _operands(201, 1024, 4096, 6)
+    exact, bound = _sums(x, w)
+    for ld in (1024, 1040):
+        buf = torch.randn(202, ld, generator=gen, device=DEV)
+        old = buf.clone()
+        sidon.conformer.residual_gemm(buf[:201, :1024], x, w)
+        want = old[:201, :1024].double() + exact
+        scale = want.abs() + exact.abs() + 1
+        assert ((buf[:201, :1024].double() - want).abs() <= bound + 9 * 2.0 ** -24 * scale).all()
+        assert torch.equal(buf[201], old[201]) and torch.equal(buf[:, 1024:], old[:, 1024:])

@@ -1,0 +1,53 @@
+"""Argument checks of the tiled GEMM's entry points: fake aligned addresses,
+each case wrong in one argument, refused before any HIP call (no GPU needed)."""
+
+from __future__ import annotations
+
+import pytest
+
+
+@pytest.mark.parametrize("over,code", [
+    (dict(x=None), -1), (dict(y=None), -1), (dict(C=48), -2), (dict(C=0), -2), (dict(K=96), -2), (dict(M=0), -2),
+    (dict(ldx=1000), -3), (dict(ldy=1023), -3), (dict(ldw=1028), -3), (dict(x=24), -4), (dict(y=40), -4),
+    (dict(M=1 << 21, ldx=1024), -2), (dict(x=1 << 30, y=(1 << 30) + 64), -2), (dict(w=1 << 30, y=(1 << 30) + 64), -2),
+])
+def test_glu_projection_rejects_bad_arguments(sidon, over, code):
+    a = dict(x=1 << 40, ldx=1024, w=1 << 41, ldw=1024, y=1 << 42, ldy=1024, M=750, C=1024, K=1024)
+    a.update(over)
+    lib = sidon._lib.load()
+    assert lib.sidon_gemm_glu(a["x"], a["ldx"], a["w"], a["ldw"], a["y"], a["ldy"], a["M"], a["C"], a["K"],
+                              None) == code
+    assert lib.sidon_last_error().decode()
+
+
+@pytest.mark.parametrize("over,code", [
+    (dict(part=None), -1), (dict(N=96), -2), (dict(K=192), -2), (dict(M=0), -2), (dict(ldx=4000), -3),
+    (dict(ldw=4100), -3), (dict(x=8), -4), (dict(part=8), -4),
+])
+def test_partial_projection_rejects_bad_arguments(sidon, over, code):
+    a = dict(x=1 << 40, ldx=4096, w=1 << 41, ldw=4096, part=1 << 42, elems=1 << 40, M=750, N=1024, K=4096)
+    a.update(over)
+    lib = sidon._lib.load()
+    assert lib.sidon_gemm_part(a["x"], a["ldx"], a["w"], a["ldw"], a["part"], a["elems"], a["M"], a["N"], a["K"],
+                               None) == code
+    assert lib.sidon_last_error().decode()
+
+
+@pytest.mark.parametrize("over,code", [
+    (dict(x=None), -1), (dict(part=None), -1), (dict(n2_w=None), -1), (dict(xn=None), -1), (dict(splits=0), -2),
+    (dict(splits=9), -2), (dict(C=1022), -2), (dict(C=2052), -2), (dict(R=0), -2), (dict(part=8), -4),
+    (dict(xn=4), -4),
+])
+def test_norm_of_partials_rejects_bad_arguments(sidon, over, code):
+    a = dict(x=16, part=32, splits=4, n2_w=48, n2_b=64, xn=80, R=10, C=1024)
+    a.update(over)
+    lib = sidon._lib.load()
+    assert lib.sidon_res_norm_parts(a["x"], a["part"], a["splits"], None, None, None, 0.0, a["n2_w"], a["n2_b"], 1e-5,
+                                    a["xn"], a["R"], a["C"], None) == code
+    assert lib.sidon_last_error().decode()
+
+
+def test_partial_rows_bound_every_smaller_call(sidon):
+    """The workspace rule is monotone and never below the rows themselves."""
+    rows = [sidon._lib.load().sidon_gemm_part_rows(m) for m in (1, 150, 4800, 8192, 8193, 50000)]
+    assert rows == sorted(rows) and rows[0] == 8192 and rows[-1] == 50000
