@@ -267,6 +267,24 @@ int sidon_fbank_frames(const float* chunk, float* frames, int B, int S, sidon_st
 int sidon_fbank_logmel(const float* spec, const float* mel_w, const int* mel_lo, const int* mel_len, int max_len,
                        float* logmel, int R, sidon_stream_t stream);
 
+/*
+ * The whole front end: chunk [B, S] fp32 (zero past each item's true length,
+ * S a positive multiple of 320) -> feats [B, S / 160, 80] fp32, which is also
+ * the stacked [B, S / 320, 160].  Per 400-sample frame (hop 160, over the chunk
+ * padded by 160 zeros on each side): DC removal, pre-emphasis 0.97,
+ * window[400], 512-point real FFT, power and mel as sidon_fbank_logmel (logmel
+ * [B, S / 160, 80] fp32 is written), then sidon_fbank_normalize.  window is the
+ * Povey window times 2^15 and roots [512][2] are (cos, sin)(-2 pi k / 512), both
+ * float64: the frames are transformed in float64 and the powers rounded to
+ * fp32.  Replaces
+ * SeamlessFbank._masked, src/sidon_triton/frontend.py:218-240, with the framing
+ * matmul of :222 taken as an FFT.  workspace:
+ * sidon_fbank_workspace_bytes(B, S / 160) bytes; window and roots 16-byte aligned.
+ */
+int sidon_fbank_features(const float* chunk, const int* valid, const double* window, const double* roots,
+                         const float* mel_w, const int* mel_lo, const int* mel_len, int max_len, float* logmel,
+                         float* workspace, size_t workspace_bytes, float* feats, int B, int S, sidon_stream_t stream);
+
 /* Bytes of the workspace sidon_fbank_normalize needs for B items of F frames. */
 size_t sidon_fbank_workspace_bytes(int B, int F);
 
@@ -300,7 +318,7 @@ int sidon_fbank_normalize(const float* logmel, const int* valid, float* workspac
  * two threads) race; every word a call reads is written earlier in the same
  * call, so consecutive calls need no clearing.  The first call on a device
  * looks up the array's device address (hipGetSymbolAddress, once per device)
- * and must run outside stream capture; later calls launch three kernels and
+ * and must run outside stream capture; later calls launch two kernels and
  * nothing else (no memset, no copy), so they may be captured into a graph.
  */
 int sidon_fbank_normalize_noalloc(const float* logmel, const int* valid, float* feats, int B, int F,

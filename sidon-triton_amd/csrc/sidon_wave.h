@@ -25,4 +25,27 @@ __device__ __forceinline__ float wave_sum(float v) {
   return (lane(v, 0) + lane(v, 16)) + (lane(v, 32) + lane(v, 48));
 }
 
+// The same for float64, each half moved on its own.
+template <int kCtrl>
+__device__ __forceinline__ double dpp_mov(double x) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, x);
+  const uint32_t lo = __builtin_amdgcn_mov_dpp((int)(uint32_t)u, kCtrl, 0xf, 0xf, false);
+  const uint32_t hi = __builtin_amdgcn_mov_dpp((int)(uint32_t)(u >> 32), kCtrl, 0xf, 0xf, false);
+  return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+
+__device__ __forceinline__ double wave_sum(double v) {
+  v += dpp_mov<0xb1>(v);
+  v += dpp_mov<0x4e>(v);
+  v += dpp_mov<0x141>(v);
+  v += dpp_mov<0x140>(v);
+  auto lane = [](double x, int l) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)u, l);
+    const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), l);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+  };
+  return (lane(v, 0) + lane(v, 16)) + (lane(v, 32) + lane(v, 48));
+}
+
 }  // namespace sidon

@@ -4,19 +4,17 @@ Mirrors ``SeamlessFbank`` of src/sidon_triton/frontend.py:175-246 (the GPU
 twin of w2v-BERT 2.0's SeamlessM4T feature extractor) for chunks zero-padded
 to a bucket of S samples (S a multiple of 320) with their true lengths:
 
-  1. ``sidon_fbank_frames`` (HIP): pad (160, 160) and cut 400-sample frames
-     with hop 160 -> [B, S / 160, 400];
-  2. framing GEMM with the constant [400, 514] matrix of ``frame_transform``
-     (DC removal, pre-emphasis 0.97, Povey window, 512-point rDFT, x 2^15),
-     fp32 on rocBLAS with the kernel chosen by timing (``blas.gemm_nt``;
-     gfx950 has no reduced-precision fp32 GEMM path, so
-     the quiet bins keep full fp32, as frontend.py:178-180 requires);
-  3. ``sidon_fbank_logmel`` (HIP): power, 80 Kaldi mel bins (sparse
-     triangles), log(max(., 1.19e-7));
-  4. ``sidon_fbank_normalize`` (HIP): per-bin mean / variance (ddof 1) over
-     each item's true frames, the odd-count pad frame of 1.0, zeros after,
-     written in the stride-2 stacked layout [B, S / 320, 160].
+  1. one kernel per 400-sample frame (hop 160, padding (160, 160)): DC removal,
+     pre-emphasis 0.97, Povey window x 2^15, 512-point real FFT in float64 (so the
+     quiet bins keep at least full fp32, as frontend.py:178-180 requires), power, 80
+     Kaldi mel bins (sparse triangles), log(max(., 1.19e-7));
+  2. per-bin mean / variance (ddof 1) over each item's true frames, the
+     odd-count pad frame of 1.0, zeros after, written in the stride-2 stacked
+     layout [B, S / 320, 160].
 
+All of it is one C call, ``sidon_fbank_features`` (csrc/fbank.hip).
+``frame_transform`` is the per-frame part as one [400, 514] matrix, the form the
+reference multiplies by (:222).
 The valid rows equal the exact-length extractor's; ``valid_features`` gives
 their count (frontend.py:243-246), the encoder's ``frames``.  Given a
 workspace the call allocates nothing and can be captured into a HIP graph.
@@ -30,7 +28,6 @@ import numpy as np
 import torch
 
 from . import _lib
-from .blas import gemm_nt
 from .flexrel import _check_device_tensor, _stream_handle
 
 SAMPLE_RATE = 16_000
@@ -84,6 +81,12 @@ def frame_transform() -> torch.Tensor:
     return torch.from_numpy(np.ascontiguousarray(w.T))
 
 
+def fft_roots() -> np.ndarray:
+    """[512, 2] float64: (cos, sin) of -2 pi k / 512."""
+    angle = -2.0 * math.pi * np.arange(N_FFT, dtype=np.float64) / N_FFT
+    return np.ascontiguousarray(np.stack([np.cos(angle), np.sin(angle)], axis=1))
+
+
 def mel_banks(num_mel: int = NUM_MEL, low: float = 20.0, high: float = SAMPLE_RATE / 2) -> np.ndarray:
     """[257, num_mel] float64 Kaldi mel filters: triangles in mel space,
     mel(f) = 1127 ln(1 + f / 700), over the rFFT bin frequencies."""
@@ -124,10 +127,8 @@ class Fbank:
         if device.type == "cuda" and device.index is None:
             device = torch.device("cuda", torch.cuda.current_device())
         self.device = device
-        # Kept as [514, 400] (rows K-contiguous), the w operand of
-        # blas.gemm_nt (y = x . w^T); this order was also the faster one when
-        # the GEMM ran on hipBLASLt (57.5 against 59.6 us at a 96 s chunk).
-        self.weight_t = frame_transform().float().t().contiguous().to(device)
+        self.window = torch.from_numpy(_povey_window() * KALDI_SCALE).to(device)
+        self.roots = torch.from_numpy(fft_roots()).to(device)
         lo, length, weights = sparse_mel(mel_banks())
         self.mel_lo = torch.from_numpy(lo).to(device)
         self.mel_len = torch.from_numpy(length).to(device)
@@ -138,9 +139,7 @@ class Fbank:
         frames = samples // FRAME_SHIFT
         f32 = dict(device=self.device, dtype=torch.float32)
         nbytes = int(_lib.load().sidon_fbank_workspace_bytes(batch, frames))
-        return {"batch": batch, "samples": samples, "frames": torch.empty(batch * frames * FRAME_SIZE, **f32),
-                "spec": torch.empty(batch * frames * 2 * N_BINS, **f32),
-                "logmel": torch.empty(batch * frames * NUM_MEL, **f32),
+        return {"batch": batch, "samples": samples, "logmel": torch.empty(batch * frames * NUM_MEL, **f32),
                 "stats": torch.empty(max(4, nbytes // 4), **f32)}
 
     @torch.no_grad()
@@ -168,27 +167,18 @@ class Fbank:
             raise ValueError("the workspace is smaller than the call")
         if not chunk.is_contiguous():
             chunk = chunk.contiguous()
-        fr = ws["frames"][:batch * frames * FRAME_SIZE].view(batch * frames, FRAME_SIZE)
-        lib = _lib.load()
-        stream = _stream_handle(device)
-        with torch.cuda.device(device):
-            rc = lib.sidon_fbank_frames(chunk.data_ptr(), fr.data_ptr(), batch, samples, stream)
-        _lib.check("sidon_fbank_frames", rc)
-        spec = ws["spec"][:batch * frames * 2 * N_BINS].view(batch * frames, 2 * N_BINS)
-        gemm_nt(fr, self.weight_t, spec)
-        logmel = ws["logmel"][:batch * frames * NUM_MEL]
         if out is None:
             out = torch.empty(batch, frames // 2, 2 * NUM_MEL, device=device)
         elif (out.dtype != torch.float32 or tuple(out.shape) != (batch, frames // 2, 2 * NUM_MEL)
               or not out.is_contiguous()):
             raise ValueError("out must be a contiguous float32 [B, S / 320, 160] tensor")
-        stats = ws["stats"]
+        logmel, stats = ws["logmel"], ws["stats"]
+        lib = _lib.load()
         with torch.cuda.device(device):
-            rc = lib.sidon_fbank_logmel(spec.data_ptr(), self.mel_w.data_ptr(), self.mel_lo.data_ptr(),
-                                        self.mel_len.data_ptr(), self.mel_w.shape[1], logmel.data_ptr(),
-                                        batch * frames, stream)
-            _lib.check("sidon_fbank_logmel", rc)
-            rc = lib.sidon_fbank_normalize(logmel.data_ptr(), valid.data_ptr(), stats.data_ptr(),
-                                           stats.numel() * 4, out.data_ptr(), batch, frames, stream)
-        _lib.check("sidon_fbank_normalize", rc)
+            rc = lib.sidon_fbank_features(chunk.data_ptr(), valid.data_ptr(), self.window.data_ptr(),
+                                          self.roots.data_ptr(), self.mel_w.data_ptr(), self.mel_lo.data_ptr(),
+                                          self.mel_len.data_ptr(), self.mel_w.shape[1], logmel.data_ptr(),
+                                          stats.data_ptr(), stats.numel() * 4, out.data_ptr(), batch, samples,
+                                          _stream_handle(device))
+        _lib.check("sidon_fbank_features", rc)
         return out

@@ -1,4 +1,4 @@
-"""Argument checks of the tiled GEMM's entry points: fake aligned addresses,
+"""Argument checks of the tiled GEMM's and the one-call front end's entry points: fake aligned addresses,
 each case wrong in one argument, refused before any HIP call (no GPU needed)."""
 
 from __future__ import annotations
@@ -51,3 +51,19 @@ def test_partial_rows_bound_every_smaller_call(sidon):
     """The workspace rule is monotone and never below the rows themselves."""
     rows = [sidon._lib.load().sidon_gemm_part_rows(m) for m in (1, 150, 4800, 8192, 8193, 50000)]
     assert rows == sorted(rows) and rows[0] == 8192 and rows[-1] == 50000
+
+
+@pytest.mark.parametrize("over,code", [
+    (dict(chunk=None), -1), (dict(roots=None), -1), (dict(feats=None), -1), (dict(B=0), -2), (dict(S=1000), -2),
+    (dict(S=160), -2), (dict(max_len=0), -2), (dict(max_len=258), -2), (dict(nbytes=64), -2), (dict(feats=112), -2),
+    (dict(B=1 << 20, nbytes=1 << 40), -2), (dict(roots=8), -4), (dict(window=8), -4),
+])
+def test_front_end_rejects_bad_arguments(sidon, over, code):
+    a = dict(chunk=16, valid=32, window=48, roots=64, mel_w=80, mel_lo=96, mel_len=96, max_len=16, logmel=112,
+             work=128, nbytes=1 << 30, feats=144, B=1, S=1536000)
+    a.update(over)
+    lib = sidon._lib.load()
+    assert lib.sidon_fbank_features(a["chunk"], a["valid"], a["window"], a["roots"], a["mel_w"], a["mel_lo"],
+                                    a["mel_len"], a["max_len"], a["logmel"], a["work"], a["nbytes"], a["feats"],
+                                    a["B"], a["S"], None) == code
+    assert lib.sidon_last_error().decode()
