@@ -324,6 +324,22 @@ int sidon_fbank_normalize(const float* logmel, const int* valid, float* workspac
 int sidon_fbank_normalize_noalloc(const float* logmel, const int* valid, float* feats, int B, int F,
                                   sidon_stream_t stream);
 
+/*
+ * A bucketed call's inputs into fixed buffers, in one launch:
+ *
+ *   dst[b, i] = src[b, i] for i < counts[b], 0 for counts[b] <= i < dst_stride
+ *   out0[b] = values0[b], out1[b] = values1[b]      int32; each output optional (NULL)
+ *
+ * src and dst fp32 on the device (both NULL: only the values), src_stride and
+ * dst_stride elements per item, dst_stride a multiple of 4, dst 16-byte
+ * aligned; counts, values0 and values1 [B] are host arrays, read before the
+ * call returns (they travel as kernel arguments, so nothing waits for the
+ * stream).  The copies into the graph's buffers of
+ * src/sidon_triton/runtime.py:374-401.
+ */
+int sidon_stage_items(const float* src, int64_t src_stride, float* dst, int64_t dst_stride, const int64_t* counts,
+                      int* out0, const int* values0, int* out1, const int* values1, int B, sidon_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -12,7 +12,11 @@ Mirrors the encoder side of src/sidon_triton/runtime.py:
   * graphs keyed by (batch, bucket), captured after a warm-up on a side
     stream, drawing from one shared memory pool, least recently used evicted
     past ``max_graphs`` (:374-401, via ``graphs.BucketGraphs``);
-  * all work enqueued on a non-default compute stream (:27, :360).
+  * all work enqueued on the caller's current stream (the reference's on a
+    compute stream of its own, :27, :360): handing a call to another stream and
+    back left the GPU idle for 100 us, which is 15% of a 3 s chunk's call.
+    Calls from several streams are ordered one after another, since they share
+    the buffers.
 
 The valid rows of a bucketed run equal an exact-length run: the front end
 takes its statistics over the true frames only, the attention masks the
@@ -26,9 +30,14 @@ runtime.py:366-372 does.  The decoder is not part of this runtime.
 
 from __future__ import annotations
 
+import contextlib
+import ctypes
+
 import torch
 
+from . import _lib
 from .encoder import HipEncoder
+from .flexrel import _stream_handle
 from .frontend import BUCKET_QUANTUM, Fbank, num_features
 from .graphs import BucketGraphs
 
@@ -60,6 +69,33 @@ def bucket_samples(samples: int, max_samples: int) -> int:
     return min(max_samples, -(-samples // step) * step)
 
 
+def stage_items(src: torch.Tensor, counts, dst: torch.Tensor, outs) -> None:
+    """dst[b] = src[b, :counts[b]] and zeros after it, and for each (out, values)
+    of ``outs`` (at most two) out[b] = values[b], on the current stream without
+    waiting for its earlier work.  src [B, ...] (any device and type), dst [B, ...] fp32
+    contiguous on the device, out int32 [B] on the device, values host ints.
+    One launch when src is a contiguous fp32 tensor of dst's device; a host src
+    is copied before the call returns, so the caller may overwrite it."""
+    batch = dst.shape[0]
+    n, m = src[0].numel(), dst[0].numel()
+    direct = src.device == dst.device and src.dtype == torch.float32 and src.is_contiguous() and m % 4 == 0
+    if not direct:
+        flat = dst.view(batch, m)
+        flat[:, :n].copy_(src.reshape(batch, n), non_blocking=src.device.type != "cpu")
+        for b, count in enumerate(counts):
+            if count < m:
+                flat[b, count:].zero_()
+    args = []
+    for out, values in outs:
+        args += [out.data_ptr(), (ctypes.c_int * batch)(*values)]
+    args += [None, None] * (2 - len(outs))
+    lib = _lib.load()
+    with torch.cuda.device(dst.device):
+        rc = lib.sidon_stage_items(src.data_ptr() if direct else None, n, dst.data_ptr() if direct else None, m,
+                                   (ctypes.c_int64 * batch)(*counts), *args, batch, _stream_handle(dst.device))
+    _lib.check("sidon_stage_items", rc)
+
+
 class EncoderRuntime:
     """Encoder calls on bucketed, graph-captured, fixed-address buffers."""
 
@@ -78,13 +114,33 @@ class EncoderRuntime:
         self.workspace = encoder.workspace(b * s)
         self.use_graph = use_graph
         self.graphs = BucketGraphs(max_graphs)
-        self.compute = torch.cuda.Stream(device=device)
+        self._done = None       # event behind the last call, if it ran on a stream other than the default one
+        self._on_default = False
         self.frontend = frontend
         self.max_samples = self.max_seq * BUCKET_QUANTUM
         if frontend is not None:
             self.wave = torch.zeros(b * self.max_samples, device=device)
             self.wave_valid = torch.zeros(b, dtype=torch.int32, device=device)
             self.fbank_workspace = frontend.workspace(b, self.max_samples)
+
+    @contextlib.contextmanager
+    def _ordered(self):
+        """The call inside runs after the runtime's earlier calls, whatever
+        streams those ran on.  (A default-stream call needs no event of its own:
+        that stream lives as long as the process, so a later call on another
+        stream can still wait for it.)"""
+        device = self.encoder.device
+        stream, default = torch.cuda.current_stream(device), torch.cuda.default_stream(device)
+        if self._done is not None:
+            stream.wait_event(self._done)
+        elif self._on_default and stream != default:
+            stream.wait_stream(default)
+        try:
+            with torch.cuda.device(device):
+                yield
+        finally:
+            self._on_default = stream == default
+            self._done = None if self._on_default else stream.record_event()
 
     def bucket(self, frames: int) -> int:
         return bucket_frames(frames, self.max_seq)
@@ -103,7 +159,7 @@ class EncoderRuntime:
         """features [B, n, F] (any device; fp32) with ``frames`` valid frames
         per item (a sequence of ints, None: all n) -> hidden [B, n, C], a view
         of the runtime's buffer valid until the next call.  Enqueued on the
-        compute stream; the current stream waits for it."""
+        current stream."""
         batch, n, nfeat = features.shape
         if not 1 <= batch <= self.max_batch:
             raise ValueError(f"batch {batch} outside [1, {self.max_batch}]")
@@ -115,19 +171,13 @@ class EncoderRuntime:
         if n > self.max_seq:
             raise ValueError(f"{n} frames exceed the runtime's maximum of {self.max_seq}")
         length = self.bucket(n)
-        caller = torch.cuda.current_stream(self.encoder.device)
-        self.compute.wait_stream(caller)
-        with torch.cuda.stream(self.compute):
+        with self._ordered():
             feats, hidden = self._views(batch, length)
-            feats[:, :n].copy_(features, non_blocking=True)
-            if n < length:
-                feats[:, n:].zero_()
-            self.lens[:batch].copy_(torch.tensor(frames, dtype=torch.int32), non_blocking=False)
+            stage_items(features, [n * nfeat] * batch, feats, [(self.lens, frames)])
             if self.use_graph:
                 self.graphs.run((batch, length), lambda: self._enqueue(batch, length))
             else:
                 self._enqueue(batch, length)
-        caller.wait_stream(self.compute)
         return hidden[:, :n]
 
     def _enqueue_wave(self, batch: int, samples: int) -> None:
@@ -154,19 +204,13 @@ class EncoderRuntime:
         if n > self.max_samples:
             raise ValueError(f"{n} samples exceed the runtime's maximum of {self.max_samples}")
         bucket = bucket_samples(n, self.max_samples)
-        caller = torch.cuda.current_stream(self.encoder.device)
-        self.compute.wait_stream(caller)
-        with torch.cuda.stream(self.compute):
+        with self._ordered():
             view = self.wave[:batch * bucket].view(batch, bucket)
-            view[:, :n].copy_(wave, non_blocking=True)
-            for b, x in enumerate(samples):
-                view[b, x:].zero_()
-            self.wave_valid[:batch].copy_(torch.tensor(samples, dtype=torch.int32))
-            self.lens[:batch].copy_(torch.tensor([num_features(x) for x in samples], dtype=torch.int32))
+            stage_items(wave, samples, view,
+                        [(self.wave_valid, samples), (self.lens, [num_features(x) for x in samples])])
             if self.use_graph:
                 self.graphs.run(("wave", batch, bucket), lambda: self._enqueue_wave(batch, bucket))
             else:
                 self._enqueue_wave(batch, bucket)
-        caller.wait_stream(self.compute)
         _, hidden = self._views(batch, bucket // BUCKET_QUANTUM)
         return hidden[:, :num_features(n)]
