@@ -14,17 +14,16 @@
 //
 // causal_dw_norm maps one thread to a channel pair and one block to BT
 // consecutive frames of one batch item over all C channels.  The thread
-// keeps its 2 K taps and BT accumulator pairs in registers and walks the
-// BT + K - 1 source frames once, adding each frame's g into every output
-// frame it reaches: each g element is read once per block (plus the K - 1
-// frames of left context the block shares with its neighbour), and every
-// output frame sums its taps in order k = 0 .. K-1.  LayerNorm reduces the
-// block's BT rows at once (wavefront butterflies, then one LDS exchange).
+// keeps its 2 K taps, its channels of the BT + K - 1 source frames and BT
+// accumulator pairs in registers: each g element is read once per block (plus
+// the K - 1 frames of left context the block shares with its neighbour), and
+// every output frame sums its taps in order k = 0 .. K-1.  LayerNorm reduces
+// the block's BT rows at once.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
 
-#include <algorithm>
+#include <initializer_list>
 
 #include "sidon_encoder.h"
 #include "sidon_host.h"
@@ -42,7 +41,6 @@ typedef float f8 __attribute__((ext_vector_type(8)));
 constexpr int kMaxC = 2048;      // channels: one thread per pair, <= 1024 threads
 constexpr int kEwThreads = 256;  // glu / silu block size
 constexpr int kXcds = 8;         // accelerator complex dies of an MI355X
-constexpr int kStageRows = 4;    // causal_dw_norm: source rows each thread loads per pass
 
 // sigmoid(x) = 1 / (1 + e^-x) with the hardware exponential and reciprocal
 // (each within about 1 ulp in fp32; the results are rounded to fp16).
@@ -142,54 +140,58 @@ struct DwParams {
   _Float16* out;        // [B*T, C]
   float eps;
   int T, C;
-  int vec8;             // C % 8 == 0 and src 16-byte aligned: 8-channel tile loads
 };
 
 using sidon::wave_sum;
 
 // Sums v[t] over the block's threads for every t < BT (result in every
-// thread).  red holds BT floats per wavefront.
-template <int BT>
-__device__ __forceinline__ void block_sums(float (&v)[BT], float* red, int nwaves) {
+// thread), in wavefront order: wavefront sums to LDS, then lane t of every
+// wavefront adds the block's for row t and hands the total to the others as a
+// scalar -- one barrier, and NW LDS reads instead of BT NW per thread.
+template <int BT, int NW>
+__device__ __forceinline__ void block_sums(float (&v)[BT], float (*red)[NW], int nwaves) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
 #pragma unroll
   for (int t = 0; t < BT; ++t) v[t] = wave_sum(v[t]);
   if (lane == 0) {
 #pragma unroll
-    for (int t = 0; t < BT; ++t) red[wave * BT + t] = v[t];
+    for (int t = 0; t < BT; ++t) red[t][wave] = v[t];
   }
   __syncthreads();
+  float s = 0.f;
 #pragma unroll
-  for (int t = 0; t < BT; ++t) v[t] = 0.f;
-  for (int w = 0; w < nwaves; ++w) {
+  for (int w = 0; w < NW; ++w)
+    if (w < nwaves) s += red[min(lane, BT - 1)][w];
 #pragma unroll
-    for (int t = 0; t < BT; ++t) v[t] += red[w * BT + t];
-  }
-  __syncthreads();  // red is reused by the next reduction
+  for (int t = 0; t < BT; ++t)
+    v[t] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), t));
 }
 
 // One block: output frames [t0, t0 + BT) of one item, all C channels (tiles
-// numbered item-major over a 1-D grid).
-//   1. The block stages g of source frames t0 - (K - 1) .. t0 + BT - 1 in LDS
-//      (fp16, zeros outside [0, T)), every thread loading whole 16-byte
-//      chunks of four rows at a time from clamped (always valid) rows, so
-//      the four rows' loads are in flight together.
-//   2. Thread i owns channels 2i, 2i + 1: its 2 K taps and BT accumulator
-//      pairs sit in registers; it walks the BT + K - 1 staged frames once,
-//      adding frame j into output i through tap k = j - i, so every output
-//      sums its taps in order k = 0 .. K-1.
+// numbered item-major over a 1-D grid).  Thread i owns channels 2i, 2i + 1.
+//   1. It loads its 2 K taps, norm weights and its channels of the BT + K - 1
+//      source frames (256 bytes per wavefront and frame) straight into
+//      registers, all in flight at once, and forms g; no other thread needs
+//      its channels, so nothing is staged.
+//   2. It walks the frames once, adding frame j into output i through tap
+//      k = j - i, so every output sums its taps in order k = 0 .. K-1.
 //   3. LayerNorm over the C channels of the BT rows (two passes, block
 //      reductions), SiLU, fp16 store.
-template <int K, int BT, bool kGlu>
-__global__ void __launch_bounds__(1024) causal_dw_norm_kernel(const DwParams p) {
-  extern __shared__ __attribute__((aligned(16))) char dw_smem[];
-  __shared__ float red[16 * BT];
+// Bound by the memory round trip and the reductions at few frames per block
+// and by vector instructions at many (20 frames: 1240 FMAs, 40 SiLUs).
+// C = 1024, K = 31, us per launch from g (from h in brackets), before with a
+// tile staged in LDS, its own wait for the taps and 8 BT LDS reads per thread
+// and reduction -> now: 150 frames 7.6 -> 5.5 (9.8 -> 7.5), 750 8.7 -> 7.3 (10.7 ->
+// 9.8), 1600 11.6 -> 9.4 (14.1 -> 12.5), 3000 18.2 -> 12.0 (20.9 -> 16.1), 4800
+// 21.7 -> 17.3 (25.1 -> 22.8).
+template <int K, int BT, bool kGlu, int kMaxThreads>
+__global__ void __launch_bounds__(kMaxThreads) causal_dw_norm_kernel(const DwParams p) {
+  constexpr int NW = kMaxThreads / 64;
   constexpr int kRows = BT + K - 1;
-  _Float16* tile = reinterpret_cast<_Float16*>(dw_smem);  // [kRows][C]
+  __shared__ float red[2][BT][NW];
   const int C = p.C;
-  const int nthreads = blockDim.x;
-  const int nwaves = nthreads >> 6;
+  const int nwaves = blockDim.x >> 6;
   // Workgroups go to the 8 XCDs round-robin; give each XCD a contiguous run
   // of tiles, so the K - 1 frames a tile shares with its left neighbour are
   // usually in the same L2.
@@ -201,89 +203,52 @@ __global__ void __launch_bounds__(1024) causal_dw_norm_kernel(const DwParams p) 
   const int t0 = (tile_id - b * ntiles) * BT;
   const int s0 = t0 - (K - 1);
   const int64_t row0 = (int64_t)b * p.T;
-  const int64_t src_stride = kGlu ? 2 * (int64_t)C : (int64_t)C;
+  const int64_t stride = kGlu ? 2 * (int64_t)C : (int64_t)C;
 
-  // 1. stage g
-  {
-    const int width = p.vec8 ? 8 : 2;          // channels per chunk
-    const int cpr = C / width;                 // chunks per row
-    const int rpp = nthreads / cpr;            // rows per pass (>= 1: C / 2 <= nthreads)
-    const int r_first = threadIdx.x / cpr;
-    const int cc = (threadIdx.x - r_first * cpr) * width;
-    if (r_first < rpp) {
-      // kStageRows rows per pass: the loads of all of them are issued before
-      // any is used (rows past the tile repeat the last one and are not stored).
-      for (int r = r_first; r < kRows; r += kStageRows * rpp) {
-        if (p.vec8) {
-          h8 a[kStageRows], gate[kStageRows];
+  // 1. loads (threads past C load its last channels and are left out of the
+  // sums; frames outside [0, T) load the nearest one)
+  const bool on = 2 * (int)threadIdx.x < C;
+  const int c = on ? 2 * threadIdx.x : C - 2;
+  const _Float16* src = p.src + row0 * stride + c;
+  // 16 wavefronts per block leave each 128 registers: 8 frames at a time there.
+  constexpr int kChunk = kMaxThreads <= 512 ? kRows : 8;
+  h2 a[kChunk], gate[kGlu ? kChunk : 1];
+  auto load = [&](int j0) {
 #pragma unroll
-          for (int u = 0; u < kStageRows; ++u) {
-            const int sc = min(max(s0 + min(r + u * rpp, kRows - 1), 0), p.T - 1);
-            const _Float16* src = p.src + (row0 + sc) * src_stride + cc;
-            a[u] = *reinterpret_cast<const h8*>(src);
-            if (kGlu) gate[u] = *reinterpret_cast<const h8*>(src + C);
-          }
-#pragma unroll
-          for (int u = 0; u < kStageRows; ++u) {
-            const int rr = r + u * rpp;
-            if (rr < kRows) {
-              const int s = s0 + rr;
-              h8 g = a[u];
-              if (kGlu) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) g[e] = glu1((float)a[u][e], (float)gate[u][e]);
-              }
-              if (s < 0 || s >= p.T) g = h8{};
-              *reinterpret_cast<h8*>(tile + rr * C + cc) = g;
-            }
-          }
-        } else {
-          h2 a[kStageRows], gate[kStageRows];
-#pragma unroll
-          for (int u = 0; u < kStageRows; ++u) {
-            const int sc = min(max(s0 + min(r + u * rpp, kRows - 1), 0), p.T - 1);
-            const _Float16* src = p.src + (row0 + sc) * src_stride + cc;
-            a[u] = *reinterpret_cast<const h2*>(src);
-            if (kGlu) gate[u] = *reinterpret_cast<const h2*>(src + C);
-          }
-#pragma unroll
-          for (int u = 0; u < kStageRows; ++u) {
-            const int rr = r + u * rpp;
-            if (rr < kRows) {
-              const int s = s0 + rr;
-              h2 g = a[u];
-              if (kGlu) g = h2{glu1((float)a[u][0], (float)gate[u][0]), glu1((float)a[u][1], (float)gate[u][1])};
-              if (s < 0 || s >= p.T) g = h2{};
-              *reinterpret_cast<h2*>(tile + rr * C + cc) = g;
-            }
-          }
-        }
-      }
+    for (int j = j0; j < min(j0 + kChunk, kRows); ++j) {
+      const _Float16* at = src + min(max(s0 + j, 0), p.T - 1) * stride;
+      a[j - j0] = *reinterpret_cast<const h2*>(at);
+      if constexpr (kGlu) gate[j - j0] = *reinterpret_cast<const h2*>(at + C);
     }
-  }
-  __syncthreads();
-
-  // 2. conv
-  const int c = 2 * threadIdx.x;
-  const bool on = c < C;  // threads past C hold zeros
+  };
+  load(0);
   f2 w[K];
 #pragma unroll
-  for (int k = 0; k < K; ++k) w[k] = on ? *reinterpret_cast<const f2*>(p.dwt + (int64_t)k * C + c) : f2{0.f, 0.f};
+  for (int k = 0; k < K; ++k) w[k] = *reinterpret_cast<const f2*>(p.dwt + (int64_t)k * C + c);
+  const f2 lw = *reinterpret_cast<const f2*>(p.ln_w + c);
+  const f2 lb = *reinterpret_cast<const f2*>(p.ln_b + c);
+  __builtin_amdgcn_sched_barrier(0);  // every load so far in front of the first product
+
+  // 2. conv
   f2 acc[BT];
 #pragma unroll
   for (int t = 0; t < BT; ++t) acc[t] = f2{0.f, 0.f};
-  if (on) {
 #pragma unroll
-    for (int j = 0; j < kRows; ++j) {
-      const h2 gh = *reinterpret_cast<const h2*>(tile + j * C + c);
-      const f2 gv = {(float)gh[0], (float)gh[1]};
+  for (int j = 0; j < kRows; ++j) {
+    if (j > 0 && j % kChunk == 0) {
+      load(j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int u = j % kChunk;
+    f2 g = {(float)a[u][0], (float)a[u][1]};
+    if constexpr (kGlu) g = f2{(float)glu1(g[0], (float)gate[u][0]), (float)glu1(g[1], (float)gate[u][1])};
+    if (j < K - 1 && s0 + j < 0) g = f2{0.f, 0.f};  // uniform: left of the item
 #pragma unroll
-      for (int i = 0; i < BT; ++i) {
-        const int k = j - i;
-        if (k >= 0 && k < K) {
-          acc[i][0] = fmaf(gv[0], w[k][0], acc[i][0]);
-          acc[i][1] = fmaf(gv[1], w[k][1], acc[i][1]);
-        }
+    for (int i = 0; i < BT; ++i) {
+      const int k = j - i;
+      if (k >= 0 && k < K) {
+        acc[i][0] = fmaf(g[0], w[k][0], acc[i][0]);
+        acc[i][1] = fmaf(g[1], w[k][1], acc[i][1]);
       }
     }
   }
@@ -291,20 +256,18 @@ __global__ void __launch_bounds__(1024) causal_dw_norm_kernel(const DwParams p) 
   // 3. LayerNorm over the C channels of every row (two passes), then SiLU.
   float v[BT];
 #pragma unroll
-  for (int t = 0; t < BT; ++t) v[t] = acc[t][0] + acc[t][1];
-  block_sums<BT>(v, red, nwaves);
+  for (int t = 0; t < BT; ++t) v[t] = on ? acc[t][0] + acc[t][1] : 0.f;
+  block_sums<BT, NW>(v, red[0], nwaves);
   const float inv_c = 1.f / (float)C;
 #pragma unroll
   for (int t = 0; t < BT; ++t) {
     const float mean = v[t] * inv_c;
-    acc[t][0] = on ? acc[t][0] - mean : 0.f;
-    acc[t][1] = on ? acc[t][1] - mean : 0.f;
-    v[t] = acc[t][0] * acc[t][0] + acc[t][1] * acc[t][1];
+    acc[t][0] -= mean;
+    acc[t][1] -= mean;
+    v[t] = on ? acc[t][0] * acc[t][0] + acc[t][1] * acc[t][1] : 0.f;
   }
-  block_sums<BT>(v, red, nwaves);
+  block_sums<BT, NW>(v, red[1], nwaves);
   if (!on) return;
-  const f2 lw = *reinterpret_cast<const f2*>(p.ln_w + c);
-  const f2 lb = *reinterpret_cast<const f2*>(p.ln_b + c);
 #pragma unroll
   for (int t = 0; t < BT; ++t) {
     if (t0 + t >= p.T) continue;
@@ -315,23 +278,16 @@ __global__ void __launch_bounds__(1024) causal_dw_norm_kernel(const DwParams p) 
   }
 }
 
-constexpr int kLdsBudget = 160 * 1024;  // LDS of one CU
-
-int dw_lds_bytes(int bt, int K, int C) { return (bt + K - 1) * C * 2; }
-
 // Frames per block: the candidate that minimises (blocks per compute unit,
-// rounded up) x (staged frames per block), within the LDS of one CU.  Blocks
-// are counted per CU, not per resident slot: two blocks sharing a CU run no
-// faster than one after the other (T = 1500, C = 1024: 376 blocks of 4
-// frames, two per CU, take 15.9 us against 13.0 us for 188 blocks of 8).
-int pick_bt(int K, int B, int T, int C) {
-  static const int kCands[] = {20, 16, 8, 4};
+// rounded up) x (source frames per block).  Blocks are counted per CU, not per
+// resident slot: two blocks sharing a CU run no faster than one after the
+// other (1600 frames: 400 blocks of 4 10.3 us, 200 of 8 9.4; 150 frames: 38 of
+// 4 6.9, 150 of 1 5.5).
+int pick_bt(std::initializer_list<int> frames, int K, int B, int T) {
   int best = 0;
   long best_cost = 0;
   const int cus = sidon::compute_units();
-  for (int bt : kCands) {
-    const int lds = dw_lds_bytes(bt, K, C) + 16 * bt * 4;
-    if (lds > kLdsBudget) continue;
+  for (int bt : frames) {
     const long blocks = (long)((T + bt - 1) / bt) * B;
     const long cost = ((blocks + cus - 1) / cus) * (bt + K - 1);
     if (best == 0 || cost < best_cost) {
@@ -342,31 +298,32 @@ int pick_bt(int K, int B, int T, int C) {
   return best;
 }
 
-template <int K, int BT>
-hipError_t launch_dw_bt(const DwParams& p, int B, bool glu_input, int threads, hipStream_t stream) {
-  const dim3 grid((unsigned)(((p.T + BT - 1) / BT) * B));
-  const size_t lds = (size_t)dw_lds_bytes(BT, K, p.C);
+template <int K, int BT, int kMaxThreads>
+hipError_t launch_dw_bt(const DwParams& p, int B, bool glu_input, hipStream_t stream) {
+  const dim3 grid((unsigned)(((p.T + BT - 1) / BT) * B)), block(64 * ((p.C / 2 + 63) / 64));
   if (glu_input) {
-    auto fn = causal_dw_norm_kernel<K, BT, true>;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(fn, grid, dim3(threads), lds, stream, p);
+    hipLaunchKernelGGL((causal_dw_norm_kernel<K, BT, true, kMaxThreads>), grid, block, 0, stream, p);
   } else {
-    auto fn = causal_dw_norm_kernel<K, BT, false>;
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    hipLaunchKernelGGL(fn, grid, dim3(threads), lds, stream, p);
+    hipLaunchKernelGGL((causal_dw_norm_kernel<K, BT, false, kMaxThreads>), grid, block, 0, stream, p);
   }
   return hipGetLastError();
 }
 
 template <int K>
 hipError_t launch_dw(const DwParams& p, int B, bool glu_input, hipStream_t stream) {
-  const int threads = 64 * ((p.C / 2 + 63) / 64);
-  switch (pick_bt(K, B, p.T, p.C)) {
-    case 20: return launch_dw_bt<K, 20>(p, B, glu_input, threads, stream);
-    case 16: return launch_dw_bt<K, 16>(p, B, glu_input, threads, stream);
-    case 8: return launch_dw_bt<K, 8>(p, B, glu_input, threads, stream);
-    case 4: return launch_dw_bt<K, 4>(p, B, glu_input, threads, stream);
-    default: return hipErrorInvalidConfiguration;
+  if (p.C > 1024) {
+    return pick_bt({8, 4}, K, B, p.T) == 8 ? launch_dw_bt<K, 8, 1024>(p, B, glu_input, stream)
+                                           : launch_dw_bt<K, 4, 1024>(p, B, glu_input, stream);
+  }
+  switch (pick_bt({20, 16, 12, 8, 6, 4, 2, 1}, K, B, p.T)) {
+    case 20: return launch_dw_bt<K, 20, 512>(p, B, glu_input, stream);
+    case 16: return launch_dw_bt<K, 16, 512>(p, B, glu_input, stream);
+    case 12: return launch_dw_bt<K, 12, 512>(p, B, glu_input, stream);
+    case 8: return launch_dw_bt<K, 8, 512>(p, B, glu_input, stream);
+    case 6: return launch_dw_bt<K, 6, 512>(p, B, glu_input, stream);
+    case 4: return launch_dw_bt<K, 4, 512>(p, B, glu_input, stream);
+    case 2: return launch_dw_bt<K, 2, 512>(p, B, glu_input, stream);
+    default: return launch_dw_bt<K, 1, 512>(p, B, glu_input, stream);
   }
 }
 
@@ -440,8 +397,7 @@ SIDON_API int sidon_causal_dw_norm(const void* src, int glu_input, const float* 
     return fail(SIDON_E_ALIGN, "fp32 tensors must be 8-byte aligned");
   int rc;
   if ((rc = sidon::check_device())) return rc;
-  const int vec8 = C % 8 == 0 && aligned(src, 16);
-  const DwParams p{static_cast<const _Float16*>(src), dwt, ln_w, ln_b, static_cast<_Float16*>(out), eps, T, C, vec8};
+  const DwParams p{static_cast<const _Float16*>(src), dwt, ln_w, ln_b, static_cast<_Float16*>(out), eps, T, C};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const bool g = glu_input != 0;
   hipError_t err;

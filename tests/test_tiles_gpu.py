@@ -156,3 +156,26 @@ def test_residual_gemm_takes_the_split_or_the_strided_stream(sidon):
         scale = want.abs() + exact.abs() + 1
         assert ((buf[:201, :1024].double() - want).abs() <= bound + 9 * 2.0 ** -24 * scale).all()
         assert torch.equal(buf[201], old[201]) and torch.equal(buf[:, 1024:], old[:, 1024:])
+
+
+@pytest.mark.parametrize("batch,t,c", [(1, 1, 2), (1, 150, 1024), (2, 250, 1024), (1, 500, 130), (3, 333, 1024),
+                                       (1, 1500, 1024), (4, 400, 1024), (1, 3001, 1024), (1, 4999, 64),
+                                       (2, 700, 1026), (1, 3000, 2048)])
+def test_conv_module_at_every_block_size(sidon, batch, t, c):
+    """Frame counts that pick each number of frames per block, ragged last
+    blocks, channel counts that leave a wavefront part empty, both widths of a
+    block: from h and from g alike, bit for bit, and against float64 torch."""
+    gen = torch.Generator(device=DEV).manual_seed(t + c)
+    h = torch.randn(batch * t, 2 * c, generator=gen, device=DEV).half()
+    taps = torch.randn(31, c, generator=gen, device=DEV) * 0.2
+    w, b = 1 + 0.1 * torch.randn(c, generator=gen, device=DEV), 0.1 * torch.randn(c, generator=gen, device=DEV)
+    g = sidon.conformer.glu(h)
+    wide = torch.full((batch * t + 1, c), 7.0, dtype=torch.float16, device=DEV)
+    got = sidon.conformer.causal_dw_norm(g, batch, taps, w, b, 1e-5, out=wide[:batch * t])
+    assert torch.equal(sidon.conformer.glu_causal_dw_norm(h, batch, taps, w, b, 1e-5), got)
+    assert (wide[batch * t] == 7).all()
+    x = torch.nn.functional.pad(g.double().view(batch, t, c), (0, 0, 30, 0))
+    y = sum(taps[k].double() * x[:, k:k + t] for k in range(31)).reshape(batch * t, c)
+    y = torch.nn.functional.silu(torch.nn.functional.layer_norm(y, (c,), w.double(), b.double(), 1e-5))
+    # fp32 sums and norm of values of a few units, one rounding to fp16
+    assert ((got.double() - y).abs() <= 2.0 ** -11 * y.abs() + 3e-5).all()
