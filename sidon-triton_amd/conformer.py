@@ -303,8 +303,11 @@ def residual_gemm(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> torch.Te
     lib = _lib.load()
     with torch.cuda.device(device):
         stream = _stream_handle(device)
-        # The pass that adds the partial sums (2-3 us) pays only for a long K.
-        splits = lib.sidon_gemm_part_splits(rows, n, k) if x.is_contiguous() and k >= 2 * n and n <= 2048 else 1
+        # A pass of its own for the partial sums pays for a long K and few rows
+        # (n = 1024, k = 4096, us, split and pass against in place: 150 rows 8.7
+        # / 13.3, 750 16.7 / 20.0, 1600 26.4 / 25.0, 3000 38 / 33.4).
+        short = rows <= 1024 and k >= 2 * n and n <= 2048 and x.is_contiguous()
+        splits = lib.sidon_gemm_part_splits(rows, n, k) if short else 1
         if splits > 1 and x.data_ptr() % 16 == 0:
             part = torch.empty(splits * rows * n, device=device)
             rc = lib.sidon_gemm_part(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), part.data_ptr(),

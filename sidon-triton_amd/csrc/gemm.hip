@@ -21,8 +21,8 @@
 // of the encoder's five projections at M = 25-4800 with weights from HBM
 // (rms 9%).  The tile with the least estimate is taken; it is 0-3% (mean per
 // projection) slower than the best one measured.  A K split costs the norm
-// behind it its partial tiles and the stream's write on top, out of the MALL
-// (4 splits at M = 750: 0.7 us for 15 MB).
+// behind it its partial tiles and the stream's write on top, at 7-11 TB/s
+// (N = 1024: 4 splits at M = 750 1.4 us, 2 at 1600 2.3, 2 at 3000 5.7).
 //
 // Measured on MI355X (weights from HBM, graph replays, us), own | library:
 //   M =                          150          750          1600         4800
@@ -90,8 +90,7 @@ struct Choice {
   double us = 0;
 };
 
-Choice choose(int M, int N, int K, int mode, int max_splits) {
-  const int cus = sidon::compute_units();
+Choice search(int M, int N, int K, int mode, int max_splits, int cus) {
   const int slices = K / 64;
   Choice best;
   for (const TileKernel& t : kTiles) {
@@ -106,11 +105,28 @@ Choice choose(int M, int N, int K, int mode, int max_splits) {
       const double nk = (double)slices / s;
       double us = 3.0 + load * (0.062 * nk * mm + 0.031 * nk + (mode <= kGlu ? 0.39 : 0.48) * mm) +
                   0.065 * (n / cus) * nk * cp;
-      if (s > 1) us += (s + 1.0) * M * N * 4.0 / 1.5e7;  // partial tiles read back, the stream written by the norm
+      if (s > 1) us += (s + 1.0) * M * N * 4.0 / 8e6;  // partial tiles read back, the stream written by the norm
       if (best.tile == nullptr || us < best.us) best = Choice{&t, s, us};
     }
   }
   return best;
+}
+
+// The search (a few microseconds) once per shape: an encoder call asks for the
+// same few again and again.  One table per thread, the newest shape kept.
+Choice choose(int M, int N, int K, int mode, int max_splits) {
+  struct Entry {
+    int M, N, K, mode, max_splits, cus;
+    Choice choice;
+  };
+  constexpr unsigned kEntries = 32;
+  static thread_local Entry table[kEntries] = {};
+  const int cus = sidon::compute_units();
+  const unsigned hash = ((unsigned)M * 2654435761u ^ (unsigned)N * 40503u ^ (unsigned)K * 97u ^ (unsigned)mode) >> 7;
+  Entry& e = table[hash % kEntries];
+  if (e.M != M || e.N != N || e.K != K || e.mode != mode || e.max_splits != max_splits || e.cus != cus)
+    e = Entry{M, N, K, mode, max_splits, cus, search(M, N, K, mode, max_splits, cus)};
+  return e.choice;
 }
 
 // Operands as the kernel's 16-byte copies and 32-bit offsets need them.
