@@ -44,7 +44,7 @@ import os
 import torch
 
 from . import _lib
-from .flexrel import _check_device_tensor, _stream_handle
+from .flexrel import _check_device_tensor, _on_device, _stream_handle
 
 # (operand dtype, output dtype) -> the C ABI's dtype code
 _DTYPES = {
@@ -103,7 +103,7 @@ def gemm_nt(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, beta: float = 0
     lib = _lib.load()
     head = (x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0))
     key = (device.index, m, n, k, x.stride(0), w.stride(0), out.stride(0), dtype, beta != 0.0)
-    with torch.cuda.device(device):
+    with _on_device(device):
         stream = _stream_handle(device)
         pin = _pinned(key) if key not in _tuned else None
         if pin is not None:

@@ -32,7 +32,7 @@ import ctypes
 import torch
 
 from . import _lib
-from .flexrel import _check_device_tensor, _stream_handle
+from .flexrel import _check_device_tensor, _on_device, _stream_handle
 
 
 def _fp16_rows(name, t, device, cols=None):
@@ -55,7 +55,7 @@ def glu(h: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
     else:
         _fp16_rows("out", out, device, c)
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib.sidon_glu(h.data_ptr(), out.data_ptr(), rows, c, _stream_handle(device))
     _lib.check("sidon_glu", rc)
     return out
@@ -68,7 +68,7 @@ def silu_(h: torch.Tensor) -> torch.Tensor:
     if h.dtype != torch.float16 or not h.is_contiguous():
         raise ValueError("h must be a contiguous float16 tensor")
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib.sidon_silu(h.data_ptr(), h.numel(), _stream_handle(device))
     _lib.check("sidon_silu", rc)
     return h
@@ -96,7 +96,7 @@ def _dw(src, glu_input, batch, dwt, ln_w, ln_b, eps, out):
         if out.shape[0] != rows:
             raise ValueError("out must have the input's rows")
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib.sidon_causal_dw_norm(src.data_ptr(), int(glu_input), dwt.data_ptr(), ln_w.data_ptr(),
                                       ln_b.data_ptr(), ctypes.c_float(float(eps)), out.data_ptr(), batch,
                                       rows // batch, c, dwt.shape[0], _stream_handle(device))
@@ -127,7 +127,7 @@ def linear_silu_preferred(rows: int, n: int, k: int, device=None) -> bool:
     ``silu_(torch.addmm(...))`` for x [rows, k], w [n, k] on ``device`` (past
     ``linear_silu_lt``'s own kernel, where 320 x 256 tiles fill >= 4/5 of the
     CUs in every round; at n = 4096, k = 1024 that is rows > 3840 on 256 CUs)."""
-    with torch.cuda.device(device):
+    with _on_device(device):
         return bool(_lib.load().sidon_gemm_bias_act_preferred(rows, n, k))
 
 
@@ -161,7 +161,7 @@ def linear_silu(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, out: t
     device = x.device
     rows, n, k, out = _linear_args(x, w, b, out)
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib.sidon_gemm_bias_act(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
                                      None if b is None else b.data_ptr(), out.data_ptr(), out.stride(0), rows, n, k,
                                      1 if act else 0, _stream_handle(device))
@@ -180,7 +180,7 @@ def linear_silu_lt(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, out
     device = x.device
     rows, n, k, out = _linear_args(x, w, b, out)
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib.sidon_gemm_lt_act(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0),
                                    None if b is None else b.data_ptr(), out.data_ptr(), out.stride(0), rows, n, k,
                                    1 if act else 0, _stream_handle(device))
@@ -192,7 +192,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, out: torch.Tensor)
     """out = x . w^T + b, fp16 with fp32 sums: this library's GEMM kernel up to
     the sizes where it beats the library (``sidon_gemm_half_preferred``), else
     torch.addmm.  x [M, K], w [N, K], out [M, N]."""
-    with torch.cuda.device(x.device):
+    with _on_device(x.device):
         own = _lib.load().sidon_gemm_half_preferred(x.shape[0], w.shape[0], w.shape[1])
     if own:
         return linear_silu_lt(x, w, b, out=out, act=False)
@@ -224,7 +224,7 @@ def linear_glu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None
         if out.dtype != torch.float16 or tuple(out.shape) != (rows, c) or out.stride(1) != 1:
             raise ValueError(f"out must be a float16 [{rows}, {c}] tensor with rows contiguous")
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib.sidon_gemm_glu(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0),
                                 rows, c, k, _stream_handle(device))
     _lib.check("sidon_gemm_glu", rc)
@@ -240,7 +240,7 @@ def residual_gemm_fits(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> boo
 def residual_gemm_preferred(rows: int, n: int, k: int, device=None) -> bool:
     """Whether ``residual_gemm`` is expected to beat torch.addmm for a
     [rows, k], w [n, k] on ``device`` (up to 5 * 2^20 outputs)."""
-    with torch.cuda.device(device):
+    with _on_device(device):
         return bool(_lib.load().sidon_gemm_res_preferred(rows, n, k))
 
 
@@ -249,7 +249,7 @@ def residual_splits(rows: int, n: int, k: int, device=None) -> int:
     where the in-place ``residual_gemm`` is the better call, or 0 where
     torch.addmm is.  Depends on the shape and the device alone."""
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         return int(lib.sidon_gemm_part_splits(rows, n, k)) if lib.sidon_gemm_res_preferred(rows, n, k) else 0
 
 
@@ -279,7 +279,7 @@ def residual_partials(a: torch.Tensor, w: torch.Tensor, part: torch.Tensor) -> t
     if part.dtype != torch.float32 or not part.is_contiguous():
         raise ValueError("part must be a contiguous float32 tensor")
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         splits = lib.sidon_gemm_part_splits(rows, n, k)
         rc = lib.sidon_gemm_part(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), part.data_ptr(), part.numel(),
                                  rows, n, k, _stream_handle(device))
@@ -301,7 +301,7 @@ def residual_gemm(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> torch.Te
     if x.dtype != torch.float32 or tuple(x.shape) != (rows, n) or x.stride(1) != 1:
         raise ValueError(f"x must be a float32 [{rows}, {n}] tensor with rows contiguous")
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         stream = _stream_handle(device)
         # A pass of its own for the partial sums pays for a long K and few rows
         # (n = 1024, k = 4096, us, split and pass against in place: 150 rows 8.7

@@ -13,7 +13,7 @@ from __future__ import annotations
 import torch
 
 from . import _lib
-from .flexrel import HEAD_DIM, NUM_POS, _check_device_tensor, _stream_handle
+from .flexrel import HEAD_DIM, NUM_POS, _check_device_tensor, _on_device, _stream_handle
 
 
 def flexrel_attention(qkv: torch.Tensor, batch: int, heads: int, rel: torch.Tensor,
@@ -42,7 +42,7 @@ def flexrel_attention(qkv: torch.Tensor, batch: int, heads: int, rel: torch.Tens
     elif out.dtype != torch.float16 or tuple(out.shape) != (rows, hidden) or not out.is_contiguous():
         raise ValueError("out must be a contiguous float16 [B*L, H*64] tensor")
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib.sidon_flexrel_fwd_qkv(qkv.data_ptr(), rel.data_ptr(),
                                        None if lens is None else lens.data_ptr(),
                                        out.data_ptr(), batch, heads, length, _stream_handle(device))

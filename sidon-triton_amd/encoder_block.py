@@ -29,7 +29,7 @@ import torch
 from . import _lib
 from .conformer import linear, residual_gemm, residual_partials, residual_splits
 from .encoder_attention import flexrel_attention
-from .flexrel import _check_device_tensor, _stream_handle
+from .flexrel import _check_device_tensor, _on_device, _stream_handle
 
 
 def _ptr(t):
@@ -77,7 +77,7 @@ def res_norm(x: torch.Tensor, y: torch.Tensor | None = None, norm1=None, write_x
         xn = None
     lib = _lib.load()
     (n1w, n1b, e1), (n2w, n2b, e2) = norms
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib.sidon_res_norm(x.data_ptr(), _ptr(y), _ptr(bias), _ptr(n1w), _ptr(n1b), ctypes.c_float(e1),
                                 int(bool(write_x)), _ptr(n2w), _ptr(n2b), ctypes.c_float(e2), _ptr(xn),
                                 int(xn_dtype == torch.float16), rows, cols, _stream_handle(device))
@@ -124,7 +124,7 @@ def res_norm_parts(x: torch.Tensor, part: torch.Tensor, bias: torch.Tensor | Non
         raise ValueError("xn must be a contiguous float16 [R, C] tensor")
     lib = _lib.load()
     (n1w, n1b, e1), (n2w, n2b, e2) = norms
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib.sidon_res_norm_parts(x.data_ptr(), part.data_ptr(), part.shape[0], _ptr(bias), _ptr(n1w), _ptr(n1b),
                                       ctypes.c_float(e1), _ptr(n2w), _ptr(n2b), ctypes.c_float(e2), _ptr(xn), rows,
                                       cols, _stream_handle(device))

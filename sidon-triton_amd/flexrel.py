@@ -8,6 +8,8 @@ asserts), plus the optional device ``lens`` of the encoder kernel
 
 from __future__ import annotations
 
+import contextlib
+
 import torch
 
 from . import _lib
@@ -17,8 +19,24 @@ NUM_POS = LEFT + RIGHT + 1  # 73
 HEAD_DIM = 64
 
 
+# The current stream's handle without the Stream object around it (0.1 us
+# against 2.9), where this torch has it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_HERE = contextlib.nullcontext()
+
+
 def _stream_handle(device: torch.device) -> int:
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
+
+
+def _on_device(device):
+    """Context in which ``device`` (a torch.device or None) is the current one:
+    nothing where it is already, which saves a launch the 2.1 us of switching."""
+    if device is None or (isinstance(device, torch.device) and device.index == torch.cuda.current_device()):
+        return _HERE
+    return torch.cuda.device(device)
 
 
 def _check_device_tensor(name: str, t: torch.Tensor, device: torch.device) -> None:
@@ -62,7 +80,7 @@ def flexrel_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, r: torc
         if out.dtype != torch.float16 or tuple(out.shape) != tuple(q.shape) or out.stride(-1) != 1:
             raise ValueError("out must be float16 [B, H, L, 64] with a contiguous last dim")
     lib = _lib.load()
-    with torch.cuda.device(device):
+    with _on_device(device):
         rc = lib.sidon_flexrel_fwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), r.data_ptr(),
             None if lens is None else lens.data_ptr(), out.data_ptr(),

@@ -28,7 +28,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from .flexrel import _check_device_tensor, _stream_handle
+from .flexrel import _check_device_tensor, _on_device, _stream_handle
 
 SAMPLE_RATE = 16_000
 FRAME_SIZE = 400
@@ -174,7 +174,7 @@ class Fbank:
             raise ValueError("out must be a contiguous float32 [B, S / 320, 160] tensor")
         logmel, stats = ws["logmel"], ws["stats"]
         lib = _lib.load()
-        with torch.cuda.device(device):
+        with _on_device(device):
             rc = lib.sidon_fbank_features(chunk.data_ptr(), valid.data_ptr(), self.window.data_ptr(),
                                           self.roots.data_ptr(), self.mel_w.data_ptr(), self.mel_lo.data_ptr(),
                                           self.mel_len.data_ptr(), self.mel_w.shape[1], logmel.data_ptr(),

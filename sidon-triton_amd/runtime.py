@@ -37,7 +37,7 @@ import torch
 
 from . import _lib
 from .encoder import HipEncoder
-from .flexrel import _stream_handle
+from .flexrel import _on_device, _stream_handle
 from .frontend import BUCKET_QUANTUM, Fbank, num_features
 from .graphs import BucketGraphs
 
@@ -90,7 +90,7 @@ def stage_items(src: torch.Tensor, counts, dst: torch.Tensor, outs) -> None:
         args += [out.data_ptr(), (ctypes.c_int * batch)(*values)]
     args += [None, None] * (2 - len(outs))
     lib = _lib.load()
-    with torch.cuda.device(dst.device):
+    with _on_device(dst.device):
         rc = lib.sidon_stage_items(src.data_ptr() if direct else None, n, dst.data_ptr() if direct else None, m,
                                    (ctypes.c_int64 * batch)(*counts), *args, batch, _stream_handle(dst.device))
     _lib.check("sidon_stage_items", rc)
@@ -136,7 +136,7 @@ class EncoderRuntime:
         elif self._on_default and stream != default:
             stream.wait_stream(default)
         try:
-            with torch.cuda.device(device):
+            with _on_device(device):
                 yield
         finally:
             self._on_default = stream == default
