@@ -188,12 +188,23 @@ def linear_silu_lt(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor | None, out
     return out
 
 
+def tile_operand(t: torch.Tensor) -> bool:
+    """Whether the tiled GEMM kernel's 16-byte copies take t [rows, K] as an
+    operand: fp16, K contiguous, rows apart and 16-byte aligned."""
+    return (t.dtype == torch.float16 and t.dim() == 2 and t.stride(1) == 1 and t.stride(0) >= t.shape[1]
+            and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0)
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """out = x . w^T + b, fp16 with fp32 sums: this library's GEMM kernel up to
-    the sizes where it beats the library (``sidon_gemm_half_preferred``), else
-    torch.addmm.  x [M, K], w [N, K], out [M, N]."""
-    with _on_device(x.device):
-        own = _lib.load().sidon_gemm_half_preferred(x.shape[0], w.shape[0], w.shape[1])
+    the sizes where it beats the library (``sidon_gemm_half_preferred``) for
+    operands as it reads them, else torch.addmm (any strides, a broadcast b).
+    x [M, K], w [N, K], out [M, N]."""
+    own = (tile_operand(x) and tile_operand(w) and b.dtype == torch.float16 and tuple(b.shape) == (w.shape[0],)
+           and b.is_contiguous() and tuple(out.shape) == (x.shape[0], w.shape[0]) and tile_operand(out))
+    if own:
+        with _on_device(x.device):
+            own = _lib.load().sidon_gemm_half_preferred(x.shape[0], w.shape[0], w.shape[1])
     if own:
         return linear_silu_lt(x, w, b, out=out, act=False)
     return torch.addmm(b, x, w.t(), out=out)
@@ -201,7 +212,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, out: torch.Tensor)
 
 def linear_glu_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether ``linear_glu`` takes x [M, K] and w [2C, K]."""
-    return w.shape[0] % 64 == 0 and w.shape[1] % 64 == 0 and x.shape[1] == w.shape[1]
+    return (w.shape[0] % 64 == 0 and w.shape[1] % 64 == 0 and x.shape[1] == w.shape[1] and tile_operand(x)
+            and tile_operand(w))
 
 
 def linear_glu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:

@@ -37,7 +37,7 @@ import torch
 from .blas import gemm_nt
 from .conformer import (causal_dw_norm, glu_causal_dw_norm, linear, linear_glu, linear_glu_fits, linear_silu,
                         linear_silu_lt, linear_silu_preferred, partial_values, residual_gemm, residual_partials,
-                        residual_splits, silu_)
+                        residual_splits, silu_, tile_operand)
 from .encoder_attention import flexrel_attention
 from .encoder_block import res_norm, res_norm_parts
 from .flexrel import HEAD_DIM, LEFT, NUM_POS, RIGHT
@@ -254,6 +254,8 @@ class HipEncoder:
         def res(a, w, bias, norm1=None, norm2=None):
             to = xn_buf if norm2 is not None else None
             n = split[a.shape[1]]
+            if self.own_residual is None and not (tile_operand(a) and tile_operand(w)):
+                n = 0
             if n > 1:
                 return res_norm_parts(x, residual_partials(a, w, part_buf), bias=bias, norm1=norm1, norm2=norm2, xn=to)
             if n == 1:

@@ -179,3 +179,38 @@ def test_conv_module_at_every_block_size(sidon, batch, t, c):
     y = torch.nn.functional.silu(torch.nn.functional.layer_norm(y, (c,), w.double(), b.double(), 1e-5))
     # fp32 sums and norm of values of a few units, one rounding to fp16
     assert ((got.double() - y).abs() <= 2.0 ** -11 * y.abs() + 3e-5).all()
+
+
+@pytest.mark.parametrize("rows", [150, 1100])
+@pytest.mark.parametrize("layout", ["columns", "rows of 1028"])
+def test_projections_take_weights_of_any_layout(sidon, rows, layout):
+    """Weights that the tiled kernel's 16-byte copies cannot read (stored
+    transposed, or with rows no multiple of 16 bytes apart) go through
+    torch.addmm: ``linear`` within its rounding, the attention sub-blocks as on
+    packed weights up to the fp16 roundings between the stages, each a part of
+    one fp16 step of the stream."""
+    def laid(w):
+        if layout == "columns":
+            return w.t().contiguous().t()
+        return torch.nn.functional.pad(w, (0, 4))[:, :w.shape[1]]
+
+    x, w, gen = _operands(rows, 3072, 1024, rows)
+    b = (torch.randn(3072, generator=gen, device=DEV) * 0.1).half()
+    exact, bound = _sums(x, w)
+    exact = exact + b.double()
+    assert not sidon.conformer.tile_operand(laid(w)) and not sidon.conformer.linear_glu_fits(x, laid(w))
+    out = sidon.conformer.linear(x, laid(w), b, torch.empty(rows, 3072, dtype=torch.float16, device=DEV))
+    assert ((out.double() - exact).abs() <= 2.0 ** -10 * exact.abs() + bound + 2.0 ** -24).all()
+
+    layers = []
+    for _ in range(2):
+        layers.append({"attn_ln": (torch.ones(1024, device=DEV), torch.zeros(1024, device=DEV), 1e-5),
+                       "qkv_w": (torch.randn(3072, 1024, generator=gen, device=DEV) * 0.02).half(), "qkv_b": b,
+                       "rel": (torch.randn(73, 64, generator=gen, device=DEV) * 0.02).half(),
+                       "out_w": (torch.randn(1024, 1024, generator=gen, device=DEV) * 0.02).half(),
+                       "cum_bias": torch.randn(1024, generator=gen, device=DEV) * 0.02})
+    stream = torch.randn(rows, 1024, generator=gen, device=DEV)
+    want = sidon.encoder_block.attention_blocks(stream.clone(), layers, 1, 16)
+    odd = [{**p, "qkv_w": laid(p["qkv_w"]), "out_w": laid(p["out_w"])} for p in layers]
+    got = sidon.encoder_block.attention_blocks(stream.clone(), odd, 1, 16)
+    assert float((got - want).norm() / want.norm()) <= 2.0 ** -11
