@@ -299,6 +299,17 @@ def residual_partials(a: torch.Tensor, w: torch.Tensor, part: torch.Tensor) -> t
     return part.view(-1)[:splits * rows * n].view(splits, rows, n)
 
 
+def _span(t: torch.Tensor):
+    """First and past-the-last byte address of a [rows, cols] tensor with contiguous rows."""
+    first = t.data_ptr()
+    return first, first + ((t.shape[0] - 1) * t.stride(0) + t.shape[1]) * t.element_size()
+
+
+def _apart(x: torch.Tensor, *others: torch.Tensor) -> bool:
+    first, end = _span(x)
+    return all(o_end <= first or end <= o_first for o_first, o_end in map(_span, others))
+
+
 def residual_gemm(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x += a . w^T in place: x [M, N] fp32 (the residual stream), a [M, K]
     and w [N, K] fp16 with K contiguous -- the
@@ -318,7 +329,8 @@ def residual_gemm(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> torch.Te
         # A pass of its own for the partial sums pays for a long K and few rows
         # (n = 1024, k = 4096, us, split and pass against in place: 150 rows 8.7
         # / 13.3, 750 16.7 / 20.0, 1600 26.4 / 25.0, 3000 38 / 33.4).
-        short = rows <= 1024 and k >= 2 * n and n <= 2048 and x.is_contiguous()
+        # Operands that overlap x are the in-place entry's to refuse.
+        short = rows <= 1024 and k >= 2 * n and n <= 2048 and x.is_contiguous() and _apart(x, a, w)
         splits = lib.sidon_gemm_part_splits(rows, n, k) if short else 1
         if splits > 1 and x.data_ptr() % 16 == 0:
             part = torch.empty(splits * rows * n, device=device)

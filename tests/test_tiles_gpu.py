@@ -214,3 +214,15 @@ def test_projections_take_weights_of_any_layout(sidon, rows, layout):
     odd = [{**p, "qkv_w": laid(p["qkv_w"]), "out_w": laid(p["out_w"])} for p in layers]
     got = sidon.encoder_block.attention_blocks(stream.clone(), odd, 1, 16)
     assert float((got - want).norm() / want.norm()) <= 2.0 ** -11
+
+
+@pytest.mark.parametrize("rows", [150, 1100])
+def test_residual_gemm_refuses_operands_in_the_stream(sidon, rows):
+    """On the split route and in place alike; touching ranges do not overlap."""
+    buf = torch.zeros(rows * 1024 + rows * 2048 + 64, device=DEV)
+    x = buf[:rows * 1024].view(rows, 1024)
+    w = torch.zeros(1024, 4096, dtype=torch.float16, device=DEV)
+    with pytest.raises(RuntimeError, match="overlap"):
+        sidon.conformer.residual_gemm(x, buf[rows * 1024 - 4:][:rows * 2048].view(torch.float16).view(rows, 4096), w)
+    sidon.conformer.residual_gemm(x, buf[rows * 1024:][:rows * 2048].view(torch.float16).view(rows, 4096), w)
+    assert (buf == 0).all()
