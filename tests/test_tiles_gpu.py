@@ -210,9 +210,9 @@ def test_projections_take_weights_of_any_layout(sidon, rows, layout):
                        "out_w": (torch.randn(1024, 1024, generator=gen, device=DEV) * 0.02).half(),
                        "cum_bias": torch.randn(1024, generator=gen, device=DEV) * 0.02})
     stream = torch.randn(rows, 1024, generator=gen, device=DEV)
-    want = sidon.encoder_block.attention_blocks(stream.clone(), layers, 1, 16)
+    want = sidon.encoder_block.attention_blocks(stream.clone(), layers, 1, 16, None)
     odd = [{**p, "qkv_w": laid(p["qkv_w"]), "out_w": laid(p["out_w"])} for p in layers]
-    got = sidon.encoder_block.attention_blocks(stream.clone(), odd, 1, 16)
+    got = sidon.encoder_block.attention_blocks(stream.clone(), odd, 1, 16, None)
     assert float((got - want).norm() / want.norm()) <= 2.0 ** -11
 
 
