@@ -87,6 +87,13 @@ __device__ __forceinline__ void layer_norm(f4 (&v)[NC], int lane, int C, const f
 constexpr int kY = 1, kBias = 2, kNorm1 = 4, kWriteX = 8, kNorm2 = 16, kFp16 = 32, kFull = 64;
 constexpr int kModeBiasNorm = kBias | kNorm2 | kFp16 | kFull;                     // x + b -> LN2 (fp16)
 constexpr int kModeFinal = kBias | kNorm1 | kWriteX | kNorm2 | kFp16 | kFull;     // x = LN1(x + b) -> LN2
+// The ends of a stack: its first norm, its last norm, its last bias (in the
+// general form 11 us per launch at 4800 rows against 7 for a fixed one; the
+// feed-forward step of 3000 rows with a first norm 67.0 -> 65.6 us, 8 attention
+// sub-blocks of 1037 rows 317.3 -> 314.8).
+constexpr int kModeFirst = kNorm2 | kFp16 | kFull;                                // LN2(x) (fp16)
+constexpr int kModeLast = kBias | kNorm1 | kWriteX | kFull;                       // x = LN1(x + b)
+constexpr int kModeAdd = kBias | kWriteX | kFull;                                 // x = x + b
 
 template <int NC, int kMode>
 __global__ void __launch_bounds__(64 * kRowsPerBlock) res_norm_kernel(const RNParams p) {
@@ -267,6 +274,12 @@ hipError_t launch(const RNParams& p, hipStream_t stream) {
     hipLaunchKernelGGL((res_norm_kernel<NC, kModeBiasNorm>), dim3(blocks), dim3(64 * kRowsPerBlock), 0, stream, p);
   } else if (mode == kModeFinal) {
     hipLaunchKernelGGL((res_norm_kernel<NC, kModeFinal>), dim3(blocks), dim3(64 * kRowsPerBlock), 0, stream, p);
+  } else if (mode == kModeFirst) {
+    hipLaunchKernelGGL((res_norm_kernel<NC, kModeFirst>), dim3(blocks), dim3(64 * kRowsPerBlock), 0, stream, p);
+  } else if (mode == kModeLast) {
+    hipLaunchKernelGGL((res_norm_kernel<NC, kModeLast>), dim3(blocks), dim3(64 * kRowsPerBlock), 0, stream, p);
+  } else if (mode == kModeAdd) {
+    hipLaunchKernelGGL((res_norm_kernel<NC, kModeAdd>), dim3(blocks), dim3(64 * kRowsPerBlock), 0, stream, p);
   } else {
     hipLaunchKernelGGL((res_norm_kernel<NC, -1>), dim3(blocks), dim3(64 * kRowsPerBlock), 0, stream, p);
   }

@@ -226,3 +226,32 @@ def test_residual_gemm_refuses_operands_in_the_stream(sidon, rows):
         sidon.conformer.residual_gemm(x, buf[rows * 1024 - 4:][:rows * 2048].view(torch.float16).view(rows, 4096), w)
     sidon.conformer.residual_gemm(x, buf[rows * 1024:][:rows * 2048].view(torch.float16).view(rows, 4096), w)
     assert (buf == 0).all()
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 256), (5, 1024), (7, 1020), (3, 2048), (3000, 1024)])
+@pytest.mark.parametrize("form", ["first norm", "last norm", "last bias"])
+def test_res_norm_at_the_ends_of_a_stack(sidon, rows, cols, form):
+    """The forms compiled for whole 256-column chunks, and the general form beside
+    them (1020 columns), against float64."""
+    gen = torch.Generator(device=DEV).manual_seed(rows + cols)
+    x = torch.randn(rows, cols, generator=gen, device=DEV)
+    bias = torch.randn(cols, generator=gen, device=DEV)
+    w, b = (1 + 0.1 * torch.randn(cols, generator=gen, device=DEV)), 0.1 * torch.randn(cols, generator=gen, device=DEV)
+    res_norm, got = sidon.encoder_block.res_norm, x.clone()
+
+    def ln(v):
+        return torch.nn.functional.layer_norm(v, (cols,), w.double(), b.double(), 1e-5)
+
+    if form == "first norm":
+        xn = res_norm(got, norm2=(w, b, 1e-5), write_x=False)
+        want = ln(x.double())
+        # fp32 arithmetic on values of a few units; the fp16 output rounds once more
+        assert torch.equal(got, x) and xn.dtype == torch.float16
+        assert ((xn.double() - want).abs() <= 2.0 ** -11 * want.abs() + 4e-5).all()
+    elif form == "last norm":
+        res_norm(got, bias=bias, norm1=(w, b, 1e-5))
+        want = ln((x + bias).double())
+        assert ((got.double() - want).abs() <= 2e-5 * (1 + want.abs())).all()
+    else:
+        res_norm(got, bias=bias)
+        assert torch.equal(got, x + bias)
