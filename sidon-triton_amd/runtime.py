@@ -114,21 +114,25 @@ class EncoderRuntime:
         self.workspace = encoder.workspace(b * s)
         self.use_graph = use_graph
         self.graphs = BucketGraphs(max_graphs)
-        self._done = None       # event behind the last call, if it ran on a stream other than the default one
-        self._on_default = False
         self.frontend = frontend
         self.max_samples = self.max_seq * BUCKET_QUANTUM
         if frontend is not None:
             self.wave = torch.zeros(b * self.max_samples, device=device)
             self.wave_valid = torch.zeros(b, dtype=torch.int32, device=device)
             self.fbank_workspace = frontend.workspace(b, self.max_samples)
+        # The buffers' clears above come before the first call too.
+        self._mark(torch.cuda.current_stream(device), torch.cuda.default_stream(device))
+
+    def _mark(self, stream, default) -> None:
+        """Later calls wait for what ``stream`` holds now: by an event, or, for
+        the default stream, which lives as long as the process, by that stream."""
+        self._on_default = stream == default
+        self._done = None if self._on_default else stream.record_event()
 
     @contextlib.contextmanager
     def _ordered(self):
-        """The call inside runs after the runtime's earlier calls, whatever
-        streams those ran on.  (A default-stream call needs no event of its own:
-        that stream lives as long as the process, so a later call on another
-        stream can still wait for it.)"""
+        """The call inside runs after the runtime's construction and its earlier
+        calls, whatever streams those ran on."""
         device = self.encoder.device
         stream, default = torch.cuda.current_stream(device), torch.cuda.default_stream(device)
         if self._done is not None:
@@ -139,8 +143,7 @@ class EncoderRuntime:
             with _on_device(device):
                 yield
         finally:
-            self._on_default = stream == default
-            self._done = None if self._on_default else stream.record_event()
+            self._mark(stream, default)
 
     def bucket(self, frames: int) -> int:
         return bucket_frames(frames, self.max_seq)

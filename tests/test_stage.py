@@ -1,10 +1,12 @@
 """The staging of a bucketed call's inputs (csrc/stage.hip, runtime.stage_items):
 argument checks without a GPU, and on an MI355X the copies, zeros and lengths
 against torch for sources of every route (device fp32 at any alignment, other
-types, strided, host memory)."""
+types, strided, host memory); and the order of a runtime's calls over streams,
+on the host against a model of streams and events."""
 
 from __future__ import annotations
 
+import contextlib
 import ctypes
 
 import pytest
@@ -25,6 +27,70 @@ def test_stage_rejects_bad_arguments(sidon, over, code):
     assert lib.sidon_stage_items(a["src"], a["n"], a["dst"], a["m"], counts, a["out"], values, None, None, a["B"],
                                  None) == code
     assert lib.sidon_last_error().decode()
+
+
+class _Stream:
+    """What a stream's work comes after: ``seen`` holds the pieces of work that
+    are done when its next piece starts."""
+
+    def __init__(self):
+        self.seen = set()
+
+    def wait_event(self, event):
+        self.seen |= event
+
+    def wait_stream(self, other):
+        self.seen |= other.seen
+
+    def record_event(self):
+        return frozenset(self.seen)
+
+
+class _Device:
+    """Stands in for torch.cuda, the encoder and the front end of a runtime on the host."""
+
+    device = torch.device("cpu")
+    features = hidden = 4
+
+    def __init__(self, monkeypatch, runtime):
+        self.streams = {name: _Stream() for name in ("default", "a", "b")}
+        self.at, self.work, self.capturing, self.unordered = "default", 0, False, []
+        for name, value in (("current_stream", lambda device=None: self.streams[self.at]),
+                            ("default_stream", lambda device=None: self.streams["default"]),
+                            ("is_current_stream_capturing", lambda: self.capturing)):
+            monkeypatch.setattr(torch.cuda, name, value)
+        monkeypatch.setattr(runtime, "_on_device", lambda device: contextlib.nullcontext())
+        monkeypatch.setattr(runtime, "stage_items", lambda *args: self.launch())
+
+    def launch(self):
+        """A piece of work that touches the runtime's buffers, on the current stream."""
+        stream = self.streams[self.at]
+        if len(stream.seen) < self.work:
+            self.unordered.append((self.work, self.at))
+        stream.seen.add(self.work)
+        self.work += 1
+
+    def workspace(self, *sizes):
+        self.launch()      # a buffer is cleared
+        return {}
+
+    def __call__(self, *args, **kwargs):
+        self.launch()
+
+
+@pytest.mark.parametrize("order", ["default a", "a default", "a b", "b a b", "default default a", "a a b default b",
+                                   "default a default b", "b default a"])
+def test_runtime_orders_its_calls_and_its_construction(sidon, monkeypatch, order):
+    """Built on the first stream named and called on the others in turn: every
+    piece of work on the shared buffers, the constructor's clears among it,
+    comes after all earlier ones, whatever streams they are on."""
+    dev = _Device(monkeypatch, sidon.runtime)
+    dev.at, *calls = order.split()
+    rt = sidon.runtime.EncoderRuntime(dev, max_batch=1, max_seconds=2, use_graph=False, frontend=dev)
+    built = dev.work
+    for dev.at in calls:
+        rt.run(torch.zeros(1, 60, 4))
+    assert dev.work == built + 2 * len(calls) and not dev.unordered
 
 
 @pytest.mark.gpu
