@@ -132,18 +132,22 @@ class EncoderRuntime:
     @contextlib.contextmanager
     def _ordered(self):
         """The call inside runs after the runtime's construction and its earlier
-        calls, whatever streams those ran on."""
+        calls, whatever streams those ran on.  A capturing stream is refused
+        before anything is enqueued: a recording would hold this call's lengths,
+        and an event of a capture cannot be waited for outside of it."""
         device = self.encoder.device
         stream, default = torch.cuda.current_stream(device), torch.cuda.default_stream(device)
-        if self._done is not None:
-            stream.wait_event(self._done)
-        elif self._on_default and stream != default:
-            stream.wait_stream(default)
-        try:
-            with _on_device(device):
+        with _on_device(device):
+            if torch.cuda.is_current_stream_capturing():
+                raise RuntimeError("a runtime's calls cannot be captured into a graph: it keeps graphs of its own")
+            if self._done is not None:
+                stream.wait_event(self._done)
+            elif self._on_default and stream != default:
+                stream.wait_stream(default)
+            try:
                 yield
-        finally:
-            self._mark(stream, default)
+            finally:
+                self._mark(stream, default)
 
     def bucket(self, frames: int) -> int:
         return bucket_frames(frames, self.max_seq)

@@ -93,6 +93,21 @@ def test_runtime_orders_its_calls_and_its_construction(sidon, monkeypatch, order
     assert dev.work == built + 2 * len(calls) and not dev.unordered
 
 
+def test_runtime_refuses_a_capturing_stream(sidon, monkeypatch):
+    """Before it enqueues or records anything; the next call outside the capture
+    is a call like any other."""
+    dev = _Device(monkeypatch, sidon.runtime)
+    rt = sidon.runtime.EncoderRuntime(dev, max_batch=1, max_seconds=2, use_graph=False, frontend=dev)
+    built, dev.at, dev.capturing = dev.work, "a", True
+    for call in (lambda: rt.run(torch.zeros(1, 60, 4)), lambda: rt.run_wave(torch.zeros(1, 16000))):
+        with pytest.raises(RuntimeError, match="captured"):
+            call()
+    assert dev.work == built and not dev.streams["a"].seen
+    dev.capturing = False
+    rt.run(torch.zeros(1, 60, 4))
+    assert dev.work == built + 2 and not dev.unordered
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("batch,n,m", [(1, 1, 4), (1, 1023, 1024), (3, 1025, 1100), (2, 4000, 4000), (130, 37, 40)])
 @pytest.mark.parametrize("route", ["device", "offset", "double", "strided", "host"])
@@ -116,6 +131,29 @@ def test_stage_items_copy_pad_and_set(sidon, batch, n, m, route):
         want[b, :c] = data[b, :c]
     assert torch.equal(dst.cpu(), want)
     assert outs[0].tolist() == counts + [-1] and outs[1].tolist() == list(range(batch)) + [-1]
+
+
+def _runtime(sidon, max_seconds, **kw):
+    """A two-layer encoder's runtime on the GPU."""
+    from make_encoder_golden import encoder_weights
+
+    enc = sidon.encoder.HipEncoder(sidon.encoder.pack_weights(encoder_weights(2, 2, seed=9)), torch.device("cuda:0"))
+    return sidon.runtime.EncoderRuntime(enc, max_batch=1, max_seconds=max_seconds, **kw)
+
+
+@pytest.mark.gpu
+def test_runtime_call_in_a_capture_leaves_both_usable(sidon):
+    rt = _runtime(sidon, 12)
+    feats, count = torch.randn(1, 97, 160).cuda(), torch.zeros(4, device="cuda")
+    alone = rt.run(feats).clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        count.add_(1)
+        with pytest.raises(RuntimeError, match="captured"):
+            rt.run(feats)
+    for rep in range(3):
+        graph.replay()
+        assert torch.equal(rt.run(feats), alone) and (count == rep + 1).all()
 
 
 @pytest.mark.gpu
