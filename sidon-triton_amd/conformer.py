@@ -299,25 +299,13 @@ def residual_partials(a: torch.Tensor, w: torch.Tensor, part: torch.Tensor) -> t
     return part.view(-1)[:splits * rows * n].view(splits, rows, n)
 
 
-def _span(t: torch.Tensor):
-    """First and past-the-last byte address of a [rows, cols] tensor with contiguous rows."""
-    first = t.data_ptr()
-    return first, first + ((t.shape[0] - 1) * t.stride(0) + t.shape[1]) * t.element_size()
-
-
-def _apart(x: torch.Tensor, *others: torch.Tensor) -> bool:
-    first, end = _span(x)
-    return all(o_end <= first or end <= o_first for o_first, o_end in map(_span, others))
-
-
 def residual_gemm(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x += a . w^T in place: x [M, N] fp32 (the residual stream), a [M, K]
     and w [N, K] fp16 with K contiguous -- the
     ``torch.addmm(x, a, w.t(), out_dtype=torch.float32, out=x)`` of the
-    reference's res() (src/sidon_triton/triton_encoder.py:491-492).  Short
-    streams with contiguous rows take K split over workgroups and a pass that
-    adds the partial sums (allocated per call); the sums are taken in a fixed
-    order either way."""
+    reference's res() (src/sidon_triton/triton_encoder.py:491-492).  Takes no
+    memory but x; a caller with a buffer for partial sums has short streams
+    faster through ``residual_partials`` and ``encoder_block.res_norm_parts``."""
     device = x.device
     rows, n, k = _residual_operands(a, w, device)
     _check_device_tensor("x", x, device)
@@ -325,23 +313,7 @@ def residual_gemm(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> torch.Te
         raise ValueError(f"x must be a float32 [{rows}, {n}] tensor with rows contiguous")
     lib = _lib.load()
     with _on_device(device):
-        stream = _stream_handle(device)
-        # A pass of its own for the partial sums pays for a long K and few rows
-        # (n = 1024, k = 4096, us, split and pass against in place: 150 rows 8.7
-        # / 13.3, 750 16.7 / 20.0, 1600 26.4 / 25.0, 3000 38 / 33.4).
-        # Operands that overlap x are the in-place entry's to refuse.
-        short = rows <= 1024 and k >= 2 * n and n <= 2048 and x.is_contiguous() and _apart(x, a, w)
-        splits = lib.sidon_gemm_part_splits(rows, n, k) if short else 1
-        if splits > 1 and x.data_ptr() % 16 == 0:
-            part = torch.empty(splits * rows * n, device=device)
-            rc = lib.sidon_gemm_part(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), part.data_ptr(),
-                                     part.numel(), rows, n, k, stream)
-            _lib.check("sidon_gemm_part", rc)
-            rc = lib.sidon_res_norm_parts(x.data_ptr(), part.data_ptr(), splits, None, None, None, 0.0, None, None,
-                                          0.0, None, rows, n, stream)
-            _lib.check("sidon_res_norm_parts", rc)
-            return x
         rc = lib.sidon_gemm_res(a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), x.data_ptr(), x.stride(0),
-                                rows, n, k, stream)
+                                rows, n, k, _stream_handle(device))
     _lib.check("sidon_gemm_res", rc)
     return x

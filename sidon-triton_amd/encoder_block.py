@@ -7,8 +7,9 @@ Mirrors the attention part of ``TritonEncoder.__call__``
     xn  = res_norm(x, bias=running bias, norm2=attn_ln, write_x=False)   # fp16
     qkv = xn W_qkv^T + b_qkv                     (conformer.linear)
     ctx = flexrel_attention(qkv, batch, heads, rel, lens)              # this library
-    x  += ctx W_out^T                            (fp16 operands, fp32 output into the stream; short
-                                                  streams leave partial sums to the next norm)
+    x  += ctx W_out^T                            (fp16 operands, fp32 output into the stream; given
+                                                  a buffer, short streams leave partial sums to
+                                                  the next norm)
 
 The out-projection bias is not added to x by the GEMM; like the reference,
 the running sum of the biases of this and the earlier layers (``cum_bias``,
@@ -152,16 +153,17 @@ def attention_blocks(x: torch.Tensor, layers: list[dict], batch: int, heads: int
     ``qkv_b`` [3C] fp16, ``rel`` [73, 64] fp16, ``out_w`` [C, C] fp16 and
     ``cum_bias`` [C] fp32 (``running_biases`` of the out-projection biases).
     ``buffers`` (optional) holds preallocated ``xn`` [B*L, C] fp16, ``qkv``
-    [B*L, 3C] fp16, ``ctx`` [B*L, C] fp16 and ``part`` (fp32,
-    ``conformer.partial_values(B*L, C)`` values, used by short streams), so
-    the call allocates nothing and can be captured into a HIP graph; what is
-    missing is allocated once per call."""
+    [B*L, 3C] fp16 and ``ctx`` [B*L, C] fp16, so the call allocates nothing and
+    can be captured into a HIP graph; of these, what is missing is allocated
+    once per call.  With ``part`` among them (fp32,
+    ``conformer.partial_values(B*L, C)`` values) short streams split the
+    out-projection's K over workgroups, whose sums take another order."""
     rows, hid = x.shape
     buffers = buffers if buffers is not None else {}
-    splits = residual_splits(rows, hid, hid, x.device)
     part = buffers.get("part")
-    if part is None and splits > 1:
-        part = torch.empty(splits * rows * hid, device=x.device)
+    splits = residual_splits(rows, hid, hid, x.device)
+    if part is None:
+        splits = min(splits, 1)
     xn = buffers.get("xn")
     qkv = buffers.get("qkv")
     ctx = buffers.get("ctx")

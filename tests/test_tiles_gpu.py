@@ -143,9 +143,8 @@ def test_split_projections_replay_like_eager(sidon):
         _ = (start * 2).sum().item()
 
 
-def test_residual_gemm_takes_the_split_or_the_strided_stream(sidon):
-    """K = 4096 into a contiguous stream (split) and into a strided one (in
-    place): the same sums up to their order."""
+def test_residual_gemm_takes_a_contiguous_or_a_strided_stream(sidon):
+    """K = 4096 into a contiguous stream and into a strided one."""
     x, w, gen = _operands(201, 1024, 4096, 6)
     exact, bound = _sums(x, w)
     for ld in (1024, 1040):
@@ -156,6 +155,55 @@ def test_residual_gemm_takes_the_split_or_the_strided_stream(sidon):
         scale = want.abs() + exact.abs() + 1
         assert ((buf[:201, :1024].double() - want).abs() <= bound + 9 * 2.0 ** -24 * scale).all()
         assert torch.equal(buf[201], old[201]) and torch.equal(buf[:, 1024:], old[:, 1024:])
+
+
+@pytest.mark.parametrize("rows", [25, 150, 750, 1024])
+def test_residual_projections_take_no_memory(sidon, rows):
+    """``residual_gemm`` at any K, the attention sub-blocks on buffers for all
+    their results and an encoder on its workspace allocate nothing, as a capture
+    begun outside torch needs; without buffers the sub-blocks give the same bits."""
+    from make_encoder_golden import encoder_weights
+
+    def allocated():
+        return torch.cuda.memory_stats(DEV)["allocation.all.allocated"]
+
+    x, w, gen = _operands(rows, 1024, 4096, rows)
+    stream = torch.randn(rows, 1024, generator=gen, device=DEV)
+    before = allocated()
+    sidon.conformer.residual_gemm(stream, x, w)
+    sidon.conformer.residual_gemm(stream, x[:, :1024], w[:, :1024])
+    assert allocated() == before
+
+    half = dict(dtype=torch.float16, device=DEV)
+    layers = [{"attn_ln": (torch.ones(1024, device=DEV), torch.zeros(1024, device=DEV), 1e-5),
+               "qkv_w": (torch.randn(3072, 1024, generator=gen, device=DEV) * 0.02).half(),
+               "qkv_b": torch.zeros(3072, **half), "rel": torch.zeros(73, 64, **half),
+               "out_w": (torch.randn(1024, 1024, generator=gen, device=DEV) * 0.02).half(),
+               "cum_bias": torch.zeros(1024, device=DEV)} for _ in range(2)]
+    buffers = {"xn": torch.empty(rows, 1024, **half), "qkv": torch.empty(rows, 3072, **half),
+               "ctx": torch.empty(rows, 1024, **half)}
+    start = stream.clone()
+    want = sidon.encoder_block.attention_blocks(start.clone(), layers, 1, 16, None)
+    before = allocated()
+    sidon.encoder_block.attention_blocks(stream, layers, 1, 16, None, buffers)
+    assert allocated() == before and torch.equal(stream, want)
+    # sums in another order, within a part of one fp16 step of the stream
+    part = torch.full((sidon.conformer.partial_values(rows, 1024),), float("nan"), device=DEV)
+    split = start.clone()
+    before = allocated()
+    sidon.encoder_block.attention_blocks(split, layers, 1, 16, None, {**buffers, "part": part})
+    assert allocated() == before and float((split - want).norm() / want.norm()) <= 2.0 ** -11
+
+    packed = sidon.encoder.pack_weights(encoder_weights(2, 2, seed=9))
+    for own in (None, True):
+        enc = sidon.encoder.HipEncoder(packed, DEV, own_residual=own)
+        feats = torch.randn(1, rows, 160, generator=gen, device=DEV)
+        lens, out = torch.full((1,), rows, dtype=torch.int32, device=DEV), torch.empty(1, rows, enc.hidden, device=DEV)
+        ws = enc.workspace(rows)
+        enc(feats, lens, out=out, workspace=ws)       # the libraries' own first call
+        before = allocated()
+        enc(feats, lens, out=out, workspace=ws)
+        assert allocated() == before
 
 
 @pytest.mark.parametrize("batch,t,c", [(1, 1, 2), (1, 150, 1024), (2, 250, 1024), (1, 500, 130), (3, 333, 1024),
