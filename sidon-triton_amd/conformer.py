@@ -251,18 +251,21 @@ def residual_gemm_fits(x: torch.Tensor, a: torch.Tensor, w: torch.Tensor) -> boo
 
 def residual_gemm_preferred(rows: int, n: int, k: int, device=None) -> bool:
     """Whether ``residual_gemm`` is expected to beat torch.addmm for a
-    [rows, k], w [n, k] on ``device`` (up to 5 * 2^20 outputs)."""
+    [rows, k], w [n, k] on ``device`` (up to 5 * 2^20 outputs, but more than
+    2^18 where k > 2048)."""
     with _on_device(device):
         return bool(_lib.load().sidon_gemm_res_preferred(rows, n, k))
 
 
-def residual_splits(rows: int, n: int, k: int, device=None) -> int:
+def residual_splits(rows: int, n: int, k: int, device=None, part: bool = True) -> int:
     """K ranges of ``residual_partials`` for a [rows, k], w [n, k]: 2 to 8, or 1
     where the in-place ``residual_gemm`` is the better call, or 0 where
-    torch.addmm is.  Depends on the shape and the device alone."""
+    torch.addmm is.  ``part`` False: the caller has no buffer for partial sums,
+    so 1 or 0.  Depends on these and the device alone."""
     lib = _lib.load()
     with _on_device(device):
-        return int(lib.sidon_gemm_part_splits(rows, n, k)) if lib.sidon_gemm_res_preferred(rows, n, k) else 0
+        splits = int(lib.sidon_gemm_part_splits(rows, n, k)) if part else 0
+        return splits if splits > 1 else int(lib.sidon_gemm_res_preferred(rows, n, k))
 
 
 def partial_values(rows: int, n: int) -> int:

@@ -274,10 +274,15 @@ SIDON_API int sidon_gemm_glu(const void* x, int ldx, const void* w, int ldw, voi
 
 SIDON_API int sidon_gemm_res_fits(int M, int N, int K) { return res_fits(M, N, K) ? 1 : 0; }
 
-// The library's kernels were slower at every measured M of the encoder's two
-// residual shapes (25-4800, N = 1024); past the measured range they are kept.
+// The library's kernels were slower at the encoder's two residual shapes up to
+// 4800 rows of N = 1024, except at few outputs of a long K, where they split K
+// (us, in place | library: 1024 x 4096 150 rows 15.0 | 12.3, 225 13.3 | 12.1, 257
+// 13.5 | 14.9, x 2048 150 rows 8.2 | 9.7; 512 x 4096 400 rows 13.0 | 11.3; 2048 x
+// 4096 100 rows 13.7 | 12.7, 200 14.1 | 14.4).  Past the measured range they are
+// kept.
 SIDON_API int sidon_gemm_res_preferred(int M, int N, int K) {
-  if (!res_fits(M, N, K) || (int64_t)M * N > (int64_t)5 << 20) return 0;
+  const int64_t outputs = (int64_t)M * N;
+  if (!res_fits(M, N, K) || outputs > (int64_t)5 << 20 || (outputs <= 1 << 18 && K > 2048)) return 0;
   return sidon::check_device() == SIDON_OK ? 1 : 0;
 }
 

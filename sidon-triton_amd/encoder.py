@@ -245,9 +245,7 @@ class HipEncoder:
         # sums added by the next norm (2+), in place on this library's kernel
         # (1), or torch.addmm (0).
         if self.own_residual is None:
-            split = {k: residual_splits(rows, hid, k, device) for k in (hid, self.inter)}
-            if part_buf is None:
-                split = {k: min(n, 1) for k, n in split.items()}
+            split = {k: residual_splits(rows, hid, k, device, part_buf is not None) for k in (hid, self.inter)}
         else:
             split = dict.fromkeys((hid, self.inter), int(self.own_residual))
 

@@ -161,9 +161,7 @@ def attention_blocks(x: torch.Tensor, layers: list[dict], batch: int, heads: int
     rows, hid = x.shape
     buffers = buffers if buffers is not None else {}
     part = buffers.get("part")
-    splits = residual_splits(rows, hid, hid, x.device)
-    if part is None:
-        splits = min(splits, 1)
+    splits = residual_splits(rows, hid, hid, x.device, part is not None)
     xn = buffers.get("xn")
     qkv = buffers.get("qkv")
     ctx = buffers.get("ctx")

@@ -206,6 +206,19 @@ def test_residual_projections_take_no_memory(sidon, rows):
         assert allocated() == before
 
 
+@pytest.mark.parametrize("rows,n,k,in_place,split", [
+    (150, 1024, 4096, 0, True), (256, 1024, 4096, 0, True), (257, 1024, 4096, 1, True), (150, 1024, 2048, 1, True),
+    (512, 512, 4096, 0, True), (513, 512, 4096, 1, True), (25, 1024, 1024, 1, True), (5120, 1024, 1024, 1, False),
+    (5121, 1024, 1024, 0, False), (100, 1024, 192, 0, False)])
+def test_residual_route(sidon, rows, n, k, in_place, split):
+    """Split where a buffer is there and the cost rule splits, else in place where
+    that is the faster one, else the library."""
+    ops = sidon.conformer
+    assert ops.residual_gemm_preferred(rows, n, k, DEV) == bool(in_place)
+    assert ops.residual_splits(rows, n, k, DEV, part=False) == in_place
+    assert ops.residual_splits(rows, n, k, DEV) in (range(2, 9) if split else (in_place,))
+
+
 @pytest.mark.parametrize("batch,t,c", [(1, 1, 2), (1, 150, 1024), (2, 250, 1024), (1, 500, 130), (3, 333, 1024),
                                        (1, 1500, 1024), (4, 400, 1024), (1, 3001, 1024), (1, 4999, 64),
                                        (2, 700, 1026), (1, 3000, 2048)])
