@@ -30,6 +30,7 @@ from __future__ import annotations
 import ctypes
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from .flexrel import _check_device_tensor, _on_device, _stream_handle
@@ -195,12 +196,24 @@ def tile_operand(t: torch.Tensor) -> bool:
             and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0)
 
 
+def plain(*tensors: torch.Tensor) -> bool:
+    """Whether a kernel may stand in for a torch call with ``out=`` on these:
+    no subclass of its own behaviour, and nothing that autograd, in reverse or
+    forward mode, would follow (torch refuses ``out=`` there)."""
+    if any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in tensors):
+        return False
+    if torch.is_grad_enabled() and any(t.requires_grad for t in tensors):
+        return False
+    return (getattr(forward_ad, "_current_level", 0) < 0
+            or all(forward_ad.unpack_dual(t).tangent is None for t in tensors))
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """out = x . w^T + b, fp16 with fp32 sums: this library's GEMM kernel up to
     the sizes where it beats the library (``sidon_gemm_half_preferred``) for
     operands as it reads them, else torch.addmm (any strides, a broadcast b).
     x [M, K], w [N, K], out [M, N]."""
-    own = (tile_operand(x) and tile_operand(w) and b.dtype == torch.float16 and tuple(b.shape) == (w.shape[0],)
+    own = (plain(x, w, b, out) and tile_operand(x) and tile_operand(w) and b.dtype == torch.float16 and tuple(b.shape) == (w.shape[0],)
            and b.is_contiguous() and tuple(out.shape) == (x.shape[0], w.shape[0]) and tile_operand(out))
     if own:
         with _on_device(x.device):

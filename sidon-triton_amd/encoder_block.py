@@ -28,7 +28,7 @@ import ctypes
 import torch
 
 from . import _lib
-from .conformer import linear, residual_gemm, residual_partials, residual_splits, tile_operand
+from .conformer import linear, plain, residual_gemm, residual_partials, residual_splits, tile_operand
 from .encoder_attention import flexrel_attention
 from .flexrel import _check_device_tensor, _on_device, _stream_handle
 
@@ -172,7 +172,7 @@ def attention_blocks(x: torch.Tensor, layers: list[dict], batch: int, heads: int
         linear(xn, p["qkv_w"], p["qkv_b"], qkv)
         ctx = flexrel_attention(qkv, batch, heads, p["rel"], lens, out=ctx)
         last = i + 1 == len(layers)
-        own = splits if tile_operand(ctx) and tile_operand(p["out_w"]) else 0
+        own = splits if plain(x, ctx, p["out_w"]) and tile_operand(ctx) and tile_operand(p["out_w"]) else 0
         if own > 1 and not last:
             xn = res_norm_parts(x, residual_partials(ctx, p["out_w"], part), bias=p["cum_bias"],
                                 norm2=layers[i + 1]["attn_ln"], xn=xn)

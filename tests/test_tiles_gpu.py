@@ -27,6 +27,15 @@ def _sums(x, w):
     return exact, x.shape[1] * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
 
 
+def _block_layer(gen):
+    return {"attn_ln": (torch.ones(1024, device=DEV), torch.zeros(1024, device=DEV), 1e-5),
+            "qkv_w": (torch.randn(3072, 1024, generator=gen, device=DEV) * 0.02).half(),
+            "qkv_b": torch.zeros(3072, dtype=torch.float16, device=DEV),
+            "rel": torch.zeros(73, 64, dtype=torch.float16, device=DEV),
+            "out_w": (torch.randn(1024, 1024, generator=gen, device=DEV) * 0.02).half(),
+            "cum_bias": torch.zeros(1024, device=DEV)}
+
+
 @pytest.mark.parametrize("m,n,k", [
     (1, 64, 64), (31, 128, 64), (33, 64, 128), (65, 192, 192), (97, 4096, 256), (129, 4096, 320), (333, 4096, 128),
     (400, 4096, 1024), (500, 3072, 1024), (577, 3072, 1024), (577, 4096, 1024), (750, 3072, 1024), (751, 4096, 1024),
@@ -175,11 +184,7 @@ def test_residual_projections_take_no_memory(sidon, rows):
     assert allocated() == before
 
     half = dict(dtype=torch.float16, device=DEV)
-    layers = [{"attn_ln": (torch.ones(1024, device=DEV), torch.zeros(1024, device=DEV), 1e-5),
-               "qkv_w": (torch.randn(3072, 1024, generator=gen, device=DEV) * 0.02).half(),
-               "qkv_b": torch.zeros(3072, **half), "rel": torch.zeros(73, 64, **half),
-               "out_w": (torch.randn(1024, 1024, generator=gen, device=DEV) * 0.02).half(),
-               "cum_bias": torch.zeros(1024, device=DEV)} for _ in range(2)]
+    layers = [_block_layer(gen) for _ in range(2)]
     buffers = {"xn": torch.empty(rows, 1024, **half), "qkv": torch.empty(rows, 3072, **half),
                "ctx": torch.empty(rows, 1024, **half)}
     start = stream.clone()
@@ -275,6 +280,43 @@ def test_projections_take_weights_of_any_layout(sidon, rows, layout):
     odd = [{**p, "qkv_w": laid(p["qkv_w"]), "out_w": laid(p["out_w"])} for p in layers]
     got = sidon.encoder_block.attention_blocks(stream.clone(), odd, 1, 16, None)
     assert float((got - want).norm() / want.norm()) <= 2.0 ** -11
+
+
+@pytest.mark.parametrize("rows", [150, 1100])
+@pytest.mark.parametrize("name", ["x", "qkv_w", "qkv_b", "out_w"])
+def test_sub_blocks_refuse_what_autograd_would_follow(sidon, rows, name):
+    """The results go into given tensors: as torch.addmm(out=) does, the call
+    raises where a gradient or a tangent would be dropped (its form with an fp32
+    output takes a weight that requires one), and runs without gradients as on
+    plain tensors."""
+    from torch.autograd import forward_ad
+
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    layers = [_block_layer(gen) for _ in range(2)]
+    start = torch.randn(rows, 1024, generator=gen, device=DEV)
+
+    def call(change):
+        x, p = start.clone(), dict(layers[0])
+        if name == "x":
+            x = change(x)
+        else:
+            p[name] = change(p[name])
+        return sidon.encoder_block.attention_blocks(x, [p, layers[1]], 1, 16, None)
+
+    def tracked(t):
+        return t.clone().requires_grad_()
+
+    want = call(lambda t: t)
+    if name == "out_w":
+        assert float((call(tracked).detach() - want).norm() / want.norm()) <= 2.0 ** -11
+    else:
+        with pytest.raises(RuntimeError, match="automatic differentiation"):
+            call(tracked)
+    with torch.no_grad():
+        assert torch.equal(call(tracked), want)
+    with forward_ad.dual_level(), pytest.raises(NotImplementedError, match="forward AD"):
+        call(lambda t: forward_ad.make_dual(t, torch.ones_like(t)))
+    assert torch.equal(call(lambda t: torch.nn.Parameter(t, requires_grad=False)), want)
 
 
 @pytest.mark.parametrize("rows", [150, 1100])
