@@ -103,13 +103,17 @@ int sidon_gemm_bias_act(const void* x, int ldx, const void* w, int ldw, const vo
  * src/sidon_triton/triton_encoder.py:498-499 and :507-508.  Shapes: M, N,
  * K >= 1, strides >= the row lengths, every operand 2-byte aligned.  Where
  * sidon_gemm_half_preferred(M, N, K) (N and K multiples of 64, up to 9 * 2^20
- * outputs) and the operands are 16-byte aligned with strides that are
- * multiples of 8, this library's own kernel runs with the same rounding.
+ * outputs) and the operands are 16-byte aligned (the bias 8-byte) with strides
+ * that are multiples of 8, x and w each span less than 4 GiB and y lies apart
+ * from them, this library's own kernel runs with the same rounding;
+ * sidon_gemm_half_takes says so for a call's operands (pure host function).
  * Elsewhere the kernel is hipBLASLt's first heuristic choice that needs no
  * workspace, kept per problem, and the first call on a device creates its
  * hipBLASLt handle and must not run during stream capture.
  */
 int sidon_gemm_half_preferred(int M, int N, int K);
+int sidon_gemm_half_takes(const void* x, int ldx, const void* w, int ldw, const void* bias, const void* y, int ldy,
+                          int M, int N, int K);
 int sidon_gemm_lt_act(const void* x, int ldx, const void* w, int ldw, const void* bias, void* y, int ldy, int M,
                       int N, int K, int act, sidon_stream_t stream);
 

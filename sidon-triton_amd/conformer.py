@@ -210,14 +210,14 @@ def plain(*tensors: torch.Tensor) -> bool:
 
 def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """out = x . w^T + b, fp16 with fp32 sums: this library's GEMM kernel up to
-    the sizes where it beats the library (``sidon_gemm_half_preferred``) for
-    operands as it reads them, else torch.addmm (any strides, a broadcast b).
+    the sizes where it beats the library, for operands as it reads them
+    (``sidon_gemm_half_takes``), else torch.addmm (any strides, a broadcast b).
     x [M, K], w [N, K], out [M, N]."""
-    own = (plain(x, w, b, out) and tile_operand(x) and tile_operand(w) and b.dtype == torch.float16 and tuple(b.shape) == (w.shape[0],)
-           and b.is_contiguous() and tuple(out.shape) == (x.shape[0], w.shape[0]) and tile_operand(out))
-    if own:
-        with _on_device(x.device):
-            own = _lib.load().sidon_gemm_half_preferred(x.shape[0], w.shape[0], w.shape[1])
+    own = (plain(x, w, b, out) and tile_operand(x) and tile_operand(w) and x.shape[1] == w.shape[1]
+           and b.dtype == torch.float16 and tuple(b.shape) == (w.shape[0],) and b.is_contiguous()
+           and tuple(out.shape) == (x.shape[0], w.shape[0]) and tile_operand(out)
+           and _lib.load().sidon_gemm_half_takes(x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), b.data_ptr(),
+                                                 out.data_ptr(), out.stride(0), *out.shape, x.shape[1]))
     if own:
         return linear_silu_lt(x, w, b, out=out, act=False)
     return torch.addmm(b, x, w.t(), out=out)

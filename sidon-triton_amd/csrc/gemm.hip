@@ -251,6 +251,11 @@ SIDON_API int sidon_gemm_half_preferred(int M, int N, int K) {
   return sidon::check_device() == SIDON_OK ? 1 : 0;
 }
 
+SIDON_API int sidon_gemm_half_takes(const void* x, int ldx, const void* w, int ldw, const void* bias, const void* y,
+                                    int ldy, int M, int N, int K) {
+  return ldx >= K && ldw >= K && ldy >= N && sidon::gemm_half_takes(x, ldx, w, ldw, bias, y, ldy, M, N, K) ? 1 : 0;
+}
+
 SIDON_API int sidon_gemm_glu(const void* x, int ldx, const void* w, int ldw, void* y, int ldy, int M, int C, int K,
                              sidon_stream_t stream) {
   sidon::clear_error();

@@ -282,6 +282,24 @@ def test_projections_take_weights_of_any_layout(sidon, rows, layout):
     assert float((got - want).norm() / want.norm()) <= 2.0 ** -11
 
 
+@pytest.mark.parametrize("form", ["bias off 8 bytes", "output over x", "output over w"])
+def test_linear_leaves_to_torch_what_the_kernel_cannot_read(sidon, monkeypatch, form):
+    """Not to the library behind ``linear_silu_lt``, whose first call must not be
+    captured: bit for bit torch.addmm."""
+    monkeypatch.setattr(sidon.conformer, "linear_silu_lt", None)
+    x, w, gen = _operands(200, 1024, 1024, 7)
+    b = torch.randn(1026, generator=gen, device=DEV).half()
+    want = torch.addmm(b[1:1025] if "bias" in form else b[:1024], x, w.t())
+    if "bias" in form:
+        got = sidon.conformer.linear(x, w, b[1:1025], torch.empty_like(want))
+        assert torch.equal(got, want)
+    else:
+        seen = []
+        monkeypatch.setattr(torch, "addmm", lambda *args, out: seen.append(out))
+        sidon.conformer.linear(x, w, b[:1024], x if "x" in form else w[:200])
+        assert len(seen) == 1
+
+
 @pytest.mark.parametrize("rows", [150, 1100])
 @pytest.mark.parametrize("name", ["x", "qkv_w", "qkv_b", "out_w"])
 def test_sub_blocks_refuse_what_autograd_would_follow(sidon, rows, name):

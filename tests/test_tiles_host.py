@@ -20,6 +20,26 @@ def test_glu_projection_rejects_bad_arguments(sidon, over, code):
     assert lib.sidon_last_error().decode()
 
 
+@pytest.mark.parametrize("over", [
+    dict(N=96), dict(K=96), dict(M=0), dict(M=3100), dict(ldx=1000), dict(ldx=1028), dict(ldw=1020), dict(ldy=3068),
+    dict(ldy=3076), dict(x=(1 << 40) + 8), dict(w=(1 << 41) + 8), dict(y=(1 << 42) + 8), dict(bias=(1 << 43) + 4),
+    dict(bias=(1 << 43) + 2), dict(ldx=1 << 22), dict(ldw=1 << 20), dict(y=(1 << 40) + 4096), dict(y=(1 << 41) - 4096),
+])
+def test_projection_takes_only_what_the_kernel_reads(sidon, over):
+    """The answer that sends a call to the tiled kernel: each case wrong in one
+    argument (sizes, strides, alignment of each operand and of the bias, spans of
+    4 GiB, an output over an operand); the plain call, an 8-byte bias and touching
+    ranges are taken."""
+    def takes(**over):
+        a = dict(x=1 << 40, ldx=1024, w=1 << 41, ldw=1024, bias=1 << 43, y=1 << 42, ldy=3072, M=750, N=3072, K=1024)
+        a.update(over)
+        return sidon._lib.load().sidon_gemm_half_takes(a["x"], a["ldx"], a["w"], a["ldw"], a["bias"], a["y"],
+                                                       a["ldy"], a["M"], a["N"], a["K"])
+
+    assert takes() == takes(bias=(1 << 43) + 8) == takes(bias=None) == takes(y=(1 << 40) + 750 * 2048) == 1
+    assert takes(**over) == 0
+
+
 @pytest.mark.parametrize("over,code", [
     (dict(part=None), -1), (dict(N=96), -2), (dict(K=192), -2), (dict(M=0), -2), (dict(ldx=4000), -3),
     (dict(ldw=4100), -3), (dict(x=8), -4), (dict(part=8), -4),
