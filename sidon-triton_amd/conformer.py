@@ -224,9 +224,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, out: torch.Tensor)
 
 
 def linear_glu_fits(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether ``linear_glu`` takes x [M, K] and w [2C, K]."""
+    """Whether ``linear_glu`` takes x [M, K] and w [2C, K] (each spanning less
+    than 4 GiB)."""
     return (w.shape[0] % 64 == 0 and w.shape[1] % 64 == 0 and x.shape[1] == w.shape[1] and tile_operand(x)
-            and tile_operand(w))
+            and tile_operand(w) and all(2 * t.shape[0] * t.stride(0) < 1 << 32 for t in (x, w)))
 
 
 def linear_glu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:

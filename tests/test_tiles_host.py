@@ -4,6 +4,7 @@ each case wrong in one argument, refused before any HIP call (no GPU needed)."""
 from __future__ import annotations
 
 import pytest
+import torch
 
 
 @pytest.mark.parametrize("over,code", [
@@ -18,6 +19,16 @@ def test_glu_projection_rejects_bad_arguments(sidon, over, code):
     assert lib.sidon_gemm_glu(a["x"], a["ldx"], a["w"], a["ldw"], a["y"], a["ldy"], a["M"], a["C"], a["K"],
                               None) == code
     assert lib.sidon_last_error().decode()
+
+
+def test_glu_projection_declines_operands_of_4_gib(sidon):
+    """So that the encoder's pointwise conv takes its general route there."""
+    def rows(m, ld=1024):
+        return torch.empty(m, ld, dtype=torch.float16, device="meta")[:, :1024]
+
+    fits = sidon.conformer.linear_glu_fits
+    assert fits(rows((1 << 21) - 1), rows(2048)) and fits(rows(1024, 1 << 20), rows(2048))
+    assert not fits(rows(1 << 21), rows(2048)) and not fits(rows(750), rows(2048, 1 << 20))
 
 
 @pytest.mark.parametrize("over", [
