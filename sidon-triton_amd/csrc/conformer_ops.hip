@@ -172,8 +172,8 @@ __device__ __forceinline__ void block_sums(float (&v)[BT], float (*red)[NW], int
 // numbered item-major over a 1-D grid).  Thread i owns channels 2i, 2i + 1.
 //   1. It loads its 2 K taps, norm weights and its channels of the BT + K - 1
 //      source frames (256 bytes per wavefront and frame) straight into
-//      registers, all in flight at once, and forms g; no other thread needs
-//      its channels, so nothing is staged.
+//      registers, all in flight at once up to 1024 channels, and forms g; no
+//      other thread needs its channels, so nothing is staged.
 //   2. It walks the frames once, adding frame j into output i through tap
 //      k = j - i, so every output sums its taps in order k = 0 .. K-1.
 //   3. LayerNorm over the C channels of the BT rows (two passes, block
@@ -210,18 +210,22 @@ __global__ void __launch_bounds__(kMaxThreads) causal_dw_norm_kernel(const DwPar
   const bool on = 2 * (int)threadIdx.x < C;
   const int c = on ? 2 * threadIdx.x : C - 2;
   const _Float16* src = p.src + row0 * stride + c;
-  // 16 wavefronts per block leave each 128 registers: 8 frames at a time there.
-  constexpr int kChunk = kMaxThreads <= 512 ? kRows : 8;
-  h2 a[kChunk], gate[kGlu ? kChunk : 1];
-  auto load = [&](int j0) {
-#pragma unroll
-    for (int j = j0; j < min(j0 + kChunk, kRows); ++j) {
-      const _Float16* at = src + min(max(s0 + j, 0), p.T - 1) * stride;
-      a[j - j0] = *reinterpret_cast<const h2*>(at);
-      if constexpr (kGlu) gate[j - j0] = *reinterpret_cast<const h2*>(at + C);
-    }
+  // Up to 8 wavefronts per block every frame is in flight at once.  More leave
+  // each 168 or 128 registers: 8 frames at a time up to 8 output frames, past
+  // that kFlight ahead of the products, each refilled as it is taken.
+  constexpr bool kRing = kMaxThreads > 512 && BT > 8;
+  constexpr int kFlight = kMaxThreads <= 512 ? kRows : !kRing || kMaxThreads <= 768 ? 8 : kGlu ? 4 : 6;
+  h2 a[kFlight], gate[kGlu ? kFlight : 1];
+  auto load = [&](int j) {
+    const _Float16* at = src + min(max(s0 + j, 0), p.T - 1) * stride;
+    a[j % kFlight] = *reinterpret_cast<const h2*>(at);
+    if constexpr (kGlu) gate[j % kFlight] = *reinterpret_cast<const h2*>(at + C);
   };
-  load(0);
+  auto load_from = [&](int j0) {
+#pragma unroll
+    for (int j = j0; j < min(j0 + kFlight, kRows); ++j) load(j);
+  };
+  load_from(0);
   f2 w[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) w[k] = *reinterpret_cast<const f2*>(p.dwt + (int64_t)k * C + c);
@@ -235,13 +239,17 @@ __global__ void __launch_bounds__(kMaxThreads) causal_dw_norm_kernel(const DwPar
   for (int t = 0; t < BT; ++t) acc[t] = f2{0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < kRows; ++j) {
-    if (j > 0 && j % kChunk == 0) {
-      load(j);
+    if (!kRing && j > 0 && j % kFlight == 0) {
+      load_from(j);
       __builtin_amdgcn_sched_barrier(0);
     }
-    const int u = j % kChunk;
+    const int u = j % kFlight;
     f2 g = {(float)a[u][0], (float)a[u][1]};
     if constexpr (kGlu) g = f2{(float)glu1(g[0], (float)gate[u][0]), (float)glu1(g[1], (float)gate[u][1])};
+    if constexpr (kRing) {
+      if (j + kFlight < kRows) load(j + kFlight);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if (j < K - 1 && s0 + j < 0) g = f2{0.f, 0.f};  // uniform: left of the item
 #pragma unroll
     for (int i = 0; i < BT; ++i) {
@@ -309,12 +317,27 @@ hipError_t launch_dw_bt(const DwParams& p, int B, bool glu_input, hipStream_t st
   return hipGetLastError();
 }
 
+// Past 1024 channels.  Many frames per block pay from 15 taps on, where the K - 1
+// frames in front of a block are most of its work (us from h, at most 8 frames |
+// up to 20: K = 31, C = 1536 3000 frames 31.5 | 23.8, 4800 45.3 | 28.1; C = 1600 4800
+// 54.6 | 33.6; K = 15, C = 2048 4800 38.6 | 28.4; K = 3, C = 2048 3000 16.3 | 19.1).
+template <int K, int kMaxThreads>
+hipError_t launch_dw_wide(const DwParams& p, int B, bool glu_input, hipStream_t stream) {
+  if constexpr (K >= 15) {
+    const int bt = pick_bt({20, 16, 8, 4}, K, B, p.T);
+    if (bt == 20) return launch_dw_bt<K, 20, kMaxThreads>(p, B, glu_input, stream);
+    if (bt == 16) return launch_dw_bt<K, 16, kMaxThreads>(p, B, glu_input, stream);
+    if (bt == 8) return launch_dw_bt<K, 8, kMaxThreads>(p, B, glu_input, stream);
+    return launch_dw_bt<K, 4, kMaxThreads>(p, B, glu_input, stream);
+  }
+  return pick_bt({8, 4}, K, B, p.T) == 8 ? launch_dw_bt<K, 8, kMaxThreads>(p, B, glu_input, stream)
+                                         : launch_dw_bt<K, 4, kMaxThreads>(p, B, glu_input, stream);
+}
+
 template <int K>
 hipError_t launch_dw(const DwParams& p, int B, bool glu_input, hipStream_t stream) {
-  if (p.C > 1024) {
-    return pick_bt({8, 4}, K, B, p.T) == 8 ? launch_dw_bt<K, 8, 1024>(p, B, glu_input, stream)
-                                           : launch_dw_bt<K, 4, 1024>(p, B, glu_input, stream);
-  }
+  if (p.C > 1536) return launch_dw_wide<K, 1024>(p, B, glu_input, stream);
+  if (p.C > 1024) return launch_dw_wide<K, 768>(p, B, glu_input, stream);
   switch (pick_bt({20, 16, 12, 8, 6, 4, 2, 1}, K, B, p.T)) {
     case 20: return launch_dw_bt<K, 20, 512>(p, B, glu_input, stream);
     case 16: return launch_dw_bt<K, 16, 512>(p, B, glu_input, stream);

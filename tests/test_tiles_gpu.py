@@ -224,6 +224,23 @@ def test_residual_route(sidon, rows, n, k, in_place, split):
     assert ops.residual_splits(rows, n, k, DEV) in (range(2, 9) if split else (in_place,))
 
 
+def _check_conv(sidon, batch, t, c, taps_n):
+    gen = torch.Generator(device=DEV).manual_seed(t + c)
+    h = torch.randn(batch * t, 2 * c, generator=gen, device=DEV).half()
+    taps = torch.randn(taps_n, c, generator=gen, device=DEV) * 0.2
+    w, b = 1 + 0.1 * torch.randn(c, generator=gen, device=DEV), 0.1 * torch.randn(c, generator=gen, device=DEV)
+    g = sidon.conformer.glu(h)
+    wide = torch.full((batch * t + 1, c), 7.0, dtype=torch.float16, device=DEV)
+    got = sidon.conformer.causal_dw_norm(g, batch, taps, w, b, 1e-5, out=wide[:batch * t])
+    assert torch.equal(sidon.conformer.glu_causal_dw_norm(h, batch, taps, w, b, 1e-5), got)
+    assert (wide[batch * t] == 7).all()
+    x = torch.nn.functional.pad(g.double().view(batch, t, c), (0, 0, taps_n - 1, 0))
+    y = sum(taps[k].double() * x[:, k:k + t] for k in range(taps_n)).reshape(batch * t, c)
+    y = torch.nn.functional.silu(torch.nn.functional.layer_norm(y, (c,), w.double(), b.double(), 1e-5))
+    # fp32 sums and norm of values of a few units, one rounding to fp16
+    assert ((got.double() - y).abs() <= 2.0 ** -11 * y.abs() + 3e-5).all()
+
+
 @pytest.mark.parametrize("batch,t,c", [(1, 1, 2), (1, 150, 1024), (2, 250, 1024), (1, 500, 130), (3, 333, 1024),
                                        (1, 1500, 1024), (4, 400, 1024), (1, 3001, 1024), (1, 4999, 64),
                                        (2, 700, 1026), (1, 3000, 2048)])
@@ -231,20 +248,16 @@ def test_conv_module_at_every_block_size(sidon, batch, t, c):
     """Frame counts that pick each number of frames per block, ragged last
     blocks, channel counts that leave a wavefront part empty, both widths of a
     block: from h and from g alike, bit for bit, and against float64 torch."""
-    gen = torch.Generator(device=DEV).manual_seed(t + c)
-    h = torch.randn(batch * t, 2 * c, generator=gen, device=DEV).half()
-    taps = torch.randn(31, c, generator=gen, device=DEV) * 0.2
-    w, b = 1 + 0.1 * torch.randn(c, generator=gen, device=DEV), 0.1 * torch.randn(c, generator=gen, device=DEV)
-    g = sidon.conformer.glu(h)
-    wide = torch.full((batch * t + 1, c), 7.0, dtype=torch.float16, device=DEV)
-    got = sidon.conformer.causal_dw_norm(g, batch, taps, w, b, 1e-5, out=wide[:batch * t])
-    assert torch.equal(sidon.conformer.glu_causal_dw_norm(h, batch, taps, w, b, 1e-5), got)
-    assert (wide[batch * t] == 7).all()
-    x = torch.nn.functional.pad(g.double().view(batch, t, c), (0, 0, 30, 0))
-    y = sum(taps[k].double() * x[:, k:k + t] for k in range(31)).reshape(batch * t, c)
-    y = torch.nn.functional.silu(torch.nn.functional.layer_norm(y, (c,), w.double(), b.double(), 1e-5))
-    # fp32 sums and norm of values of a few units, one rounding to fp16
-    assert ((got.double() - y).abs() <= 2.0 ** -11 * y.abs() + 3e-5).all()
+    _check_conv(sidon, batch, t, c, 31)
+
+
+@pytest.mark.parametrize("taps,t,c", [(31, 4799, 1536), (31, 3001, 1030), (31, 4801, 2048), (31, 3001, 1540),
+                                      (31, 400, 1200), (15, 4799, 1100), (15, 3001, 2046), (15, 4900, 1600),
+                                      (7, 4800, 1026), (3, 3000, 1538), (3, 150, 2048)])
+def test_conv_module_past_1024_channels(sidon, taps, t, c):
+    """20, 16, 8 and 4 frames per block on up to 12 and up to 16 wavefronts, with the
+    frames ahead of the products refilled as they are taken, or 8 at a time."""
+    _check_conv(sidon, 1, t, c, taps)
 
 
 @pytest.mark.parametrize("rows", [150, 1100])
