@@ -175,6 +175,16 @@ int sidon_gemm_part(const void* x, int ldx, const void* w, int ldw, float* part,
                     int K, sidon_stream_t stream);
 
 /*
+ * What the projections above run for x [M, K] and w [N, K] on a device of `cus`
+ * compute units: the tile's rows and columns into *bm and *bn (each optional),
+ * the K ranges returned (0: no such call).  epilogue 0: sidon_gemm_bias_act and
+ * the tiled sidon_gemm_lt_act; 1: sidon_gemm_glu (N = 2 C); 2: sidon_gemm_part
+ * (max_splits 8); 3: sidon_gemm_res; max_splits is 1 but for 2.  Pure host
+ * function.
+ */
+int sidon_gemm_choice(int M, int N, int K, int epilogue, int max_splits, int cus, int* bm, int* bn);
+
+/*
  * Plain GEMM on rocBLAS with the kernel chosen per problem by timing:
  *
  *   y[m, n] = x[m, :] . w[n, :] + beta * y[m, n]      m < M, n < N, fp32 sums

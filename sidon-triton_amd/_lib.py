@@ -50,6 +50,8 @@ SIGNATURES = {
     "sidon_gemm_half_preferred": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "sidon_gemm_half_takes": (ctypes.c_int, [_VP, ctypes.c_int, _VP, ctypes.c_int, _VP, _VP, ctypes.c_int,
                                              ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "sidon_gemm_choice": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int,
+                                         ctypes.c_int, _IP, _IP]),
     "sidon_gemm_glu": (ctypes.c_int, [_VP, ctypes.c_int, _VP, ctypes.c_int, _VP, ctypes.c_int, ctypes.c_int,
                                       ctypes.c_int, ctypes.c_int, _VP]),
     "sidon_gemm_part_splits": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),

@@ -208,6 +208,15 @@ int gemm_half(const void* x, int ldx, const void* w, int ldw, const void* bias, 
 
 }  // namespace sidon
 
+SIDON_API int sidon_gemm_choice(int M, int N, int K, int epilogue, int max_splits, int cus, int* bm, int* bn) {
+  if (M < 1 || N < 64 || N % 64 != 0 || K < 64 || K % 64 != 0 || epilogue < kHalf || epilogue > kAdd || cus < 1) return 0;
+  if (max_splits < 1 || max_splits > kMaxSplits || (epilogue != kPart && max_splits != 1)) return 0;
+  const Choice c = search(M, N, K, epilogue, max_splits, cus);
+  if (bm != nullptr) *bm = c.tile->bm;
+  if (bn != nullptr) *bn = c.tile->bn;
+  return c.splits;
+}
+
 SIDON_API int sidon_gemm_bias_act_fits(int M, int N, int K) {
   return M >= 1 && N >= 256 && N % 256 == 0 && K >= 64 && K % 64 == 0 ? 1 : 0;
 }

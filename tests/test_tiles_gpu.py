@@ -1,7 +1,8 @@
 """The tiled GEMM kernel (csrc/gemm_tile.h) through each of its epilogues, at
-sizes that reach every tile shape the rule of csrc/gemm.hip picks on 256 compute
-units, one row past and before tile edges, and at fewer K slices than ring
-buffers; and the norm that adds a split projection's partial sums (needs an
+sizes that reach every tile shape the rule of csrc/gemm.hip picks for the
+encoder's projections on 256 compute units (test_tiles_host.py holds the lists
+below to that), one row past and before tile edges, and at fewer K slices than
+ring buffers; and the norm that adds a split projection's partial sums (needs an
 MI355X)."""
 
 from __future__ import annotations
@@ -12,6 +13,26 @@ import torch
 pytestmark = pytest.mark.gpu
 
 DEV = torch.device("cuda:0")
+
+
+# (rows, columns, K) by epilogue.
+LINEAR = [
+    (1, 64, 64), (31, 128, 64), (33, 64, 128), (65, 192, 192), (97, 4096, 256), (129, 4096, 320), (333, 4096, 128),
+    (400, 4096, 1024), (500, 3072, 1024), (577, 3072, 1024), (577, 4096, 1024), (750, 3072, 1024), (751, 4096, 1024),
+    (1000, 4096, 192), (1463, 3072, 1024), (1601, 3072, 1024), (2000, 4096, 128), (2303, 4096, 1024),
+    (3000, 3072, 192), (9000, 1024, 64)]
+GLU = [(m, 2048, k) for m, k in (
+    (1, 64), (33, 128), (300, 1024), (650, 1024), (900, 192), (1000, 1024), (1463, 256), (1601, 1024), (2500, 128),
+    (3000, 1024), (3600, 192), (4200, 1024), (1025, 1024), (1279, 1024))]
+PARTS = [(1, 64, 128), (33, 1024, 4096), (97, 1024, 4096), (150, 1024, 4096), (200, 1024, 4096), (300, 1024, 4096),
+         (577, 1024, 4096), (751, 1024, 4096), (1463, 1024, 4096), (150, 1024, 1024), (400, 1024, 1024),
+         (2500, 1024, 4096), (130, 1024, 4096), (257, 1024, 4096), (479, 1024, 4096), (500, 1024, 4096),
+         (865, 1024, 4096), (1121, 1024, 4096), (1599, 1024, 4096), (2047, 1024, 4096)]
+WIDE = [(2305, 4096, 1024), (2561, 4096, 1024), (3841, 4096, 1024), (4095, 4096, 1024), (4097, 4096, 1024),
+        (4799, 4096, 1024)]
+RESIDUAL = [(m, 1024, k) for k, rows in (
+    (1024, (33, 511, 513, 1025, 1537, 1599, 1601, 1700, 2049, 2200, 2561, 3000, 3500, 4097, 4799)),
+    (4096, (150, 1000, 1100, 1537, 1601, 2049, 2081, 2500, 3073, 4097))) for m in rows]
 
 
 def _operands(m, n, k, seed):
@@ -36,11 +57,7 @@ def _block_layer(gen):
             "cum_bias": torch.zeros(1024, device=DEV)}
 
 
-@pytest.mark.parametrize("m,n,k", [
-    (1, 64, 64), (31, 128, 64), (33, 64, 128), (65, 192, 192), (97, 4096, 256), (129, 4096, 320), (333, 4096, 128),
-    (400, 4096, 1024), (500, 3072, 1024), (577, 3072, 1024), (577, 4096, 1024), (750, 3072, 1024), (751, 4096, 1024),
-    (1000, 4096, 192), (1463, 3072, 1024), (1601, 3072, 1024), (2000, 4096, 128), (2303, 4096, 1024),
-    (3000, 3072, 192), (9000, 1024, 64)])
+@pytest.mark.parametrize("m,n,k", LINEAR)
 def test_linear_matches_float64(sidon, m, n, k):
     """Bias, SiLU of the fp32 sum, one rounding: within half an fp16 step of the
     float64 value plus the fp32 sums' own bound (the SiLU's slope is below
@@ -59,13 +76,45 @@ def test_linear_matches_float64(sidon, m, n, k):
         assert (wide[:, :8] == 7).all() and (wide[:, n + 8:] == 7).all() and (wide[m] == 7).all()
 
 
-@pytest.mark.parametrize("m,k", [(1, 64), (33, 128), (300, 1024), (650, 1024), (900, 192), (1000, 1024), (1463, 256),
-                                 (1601, 1024), (2500, 128), (3000, 1024), (3600, 192), (4200, 1024)])
-def test_linear_glu_is_the_projection_then_the_glu(sidon, m, k):
+@pytest.mark.parametrize("m,n,k", WIDE)
+def test_linear_silu_matches_float64(sidon, m, n, k):
+    """The form with two roundings: the sum to fp16, within half a step plus the fp32
+    sums' bound, and its SiLU (slope below 1.1) once more."""
+    x, w, gen = _operands(m, n, k, m + n + k)
+    b = (torch.randn(n, generator=gen, device=DEV) * 0.1).half()
+    exact, bound = _sums(x, w)
+    exact = exact + b.double()
+    off = 2.0 ** -11 * exact.abs() + bound + 2.0 ** -24
+    wide = torch.full((m + 1, n + 16), 7.0, dtype=torch.float16, device=DEV)
+    out = sidon.conformer.linear_silu(x, w, b, out=wide[:m, 8:n + 8], act=False)
+    assert ((out.double() - exact).abs() <= off).all()
+    out = sidon.conformer.linear_silu(x, w, b, out=wide[:m, 8:n + 8])
+    want = torch.nn.functional.silu(exact)
+    assert ((out.double() - want).abs() <= 1.1 * off + (2.0 ** -11 + 2.0 ** -20) * want.abs() + 2.0 ** -24).all()
+    assert (wide[:, :8] == 7).all() and (wide[:, n + 8:] == 7).all() and (wide[m] == 7).all()
+
+
+@pytest.mark.parametrize("m,n,k", RESIDUAL)
+def test_residual_gemm_matches_float64(sidon, m, n, k):
+    """Into random values, each lane adding the ones it loaded: the sums' bound and
+    one more fp32 rounding; rows and columns beside the stream stay untouched."""
+    x, w, gen = _operands(m, n, k, m + k)
+    exact, bound = _sums(x, w)
+    buf = torch.randn(m + 1, n + 16, generator=gen, device=DEV)
+    old = buf.clone()
+    sidon.conformer.residual_gemm(buf[:m, 8:n + 8], x, w)
+    want = old[:m, 8:n + 8].double() + exact
+    assert ((buf[:m, 8:n + 8].double() - want).abs() <= bound + 2.0 ** -24 * want.abs()).all()
+    buf[:m, 8:n + 8] = old[:m, 8:n + 8]
+    assert torch.equal(buf, old)
+
+
+@pytest.mark.parametrize("m,n,k", GLU)
+def test_linear_glu_is_the_projection_then_the_glu(sidon, m, n, k):
     """Bit for bit what the projection followed by the GLU kernel gives: the
     same sums in the same order, the same roundings."""
-    x, w, _ = _operands(m, 2048, k, m + k)
-    h = torch.empty(m, 2048, dtype=torch.float16, device=DEV)
+    x, w, _ = _operands(m, n, k, m + k)
+    h = torch.empty(m, n, dtype=torch.float16, device=DEV)
     want = sidon.conformer.glu(sidon.conformer.linear_silu(x, w, None, out=h, act=False))
     assert torch.equal(sidon.conformer.linear_glu(x, w), want)
 
@@ -80,9 +129,7 @@ def test_linear_glu_narrow_and_strided(sidon):
     assert (wide[:, :8] == 7).all() and (wide[:, 104:] == 7).all()
 
 
-@pytest.mark.parametrize("m,n,k", [(1, 64, 128), (33, 1024, 4096), (97, 1024, 4096), (150, 1024, 4096),
-                                   (200, 1024, 4096), (300, 1024, 4096), (577, 1024, 4096), (751, 1024, 4096),
-                                   (1463, 1024, 4096), (150, 1024, 1024), (400, 1024, 1024), (2500, 1024, 4096)])
+@pytest.mark.parametrize("m,n,k", PARTS)
 def test_partials_add_up_and_join_the_stream(sidon, m, n, k):
     """The partial tiles' sum against float64, twice with the same bits; a
     buffer of ``partial_values`` holds them; the norm adds them to the stream."""

@@ -1,7 +1,10 @@
 """Argument checks of the tiled GEMM's and the one-call front end's entry points: fake aligned addresses,
-each case wrong in one argument, refused before any HIP call (no GPU needed)."""
+each case wrong in one argument, refused before any HIP call; and that the sizes of test_tiles_gpu.py
+reach every tile that the GEMM's rule picks (no GPU needed)."""
 
 from __future__ import annotations
+
+import ctypes
 
 import pytest
 import torch
@@ -98,3 +101,37 @@ def test_front_end_rejects_bad_arguments(sidon, over, code):
                                     a["mel_len"], a["max_len"], a["logmel"], a["work"], a["nbytes"], a["feats"],
                                     a["B"], a["S"], None) == code
     assert lib.sidon_last_error().decode()
+
+
+def _tiles(lib, sizes, epilogue):
+    """(rows, columns, K split or not) of the tiles that run ``sizes`` on 256 compute units."""
+    bm, bn, reached = ctypes.c_int(), ctypes.c_int(), set()
+    for m, n, k in sizes:
+        splits = lib.sidon_gemm_choice(m, n, k, epilogue, 8 if epilogue == 2 else 1, 256, bm, bn)
+        assert splits >= 1
+        reached.add((bm.value, bn.value, splits > 1))
+    return reached
+
+
+# epilogue, (N, K, rows): the encoder's projections over chunks up to 96 s and
+# batches past that, as far as each one's route goes (the partial sums' single
+# ranges are the in-place epilogue's rows).
+@pytest.mark.parametrize("epilogue,projections,lists", [
+    (0, [(3072, 1024, 3072), (4096, 1024, 9600)], ["LINEAR", "WIDE"]), (1, [(2048, 1024, 9600)], ["GLU"]),
+    (2, [(1024, 1024, 512), (1024, 4096, 2560)], ["PARTS"]), (3, [(1024, 1024, 5120), (1024, 4096, 5120)], ["RESIDUAL"]),
+])
+def test_every_tile_of_the_projections_is_tested(sidon, epilogue, projections, lists):
+    """A refit of the cost rule that moves a shape shows here."""
+    import test_tiles_gpu
+
+    lib = sidon._lib.load()
+    wanted = _tiles(lib, [(m, n, k) for n, k, rows in projections for m in range(1, rows + 1)], epilogue)
+    tested = _tiles(lib, [size for name in lists for size in getattr(test_tiles_gpu, name)], epilogue)
+    assert wanted <= tested, sorted(wanted - tested)
+
+
+@pytest.mark.parametrize("args", [(0, 64, 64, 0, 1, 256), (1, 96, 64, 0, 1, 256), (1, 64, 96, 0, 1, 256),
+                                  (1, 64, 64, 4, 1, 256), (1, 64, 64, -1, 1, 256), (1, 64, 64, 0, 2, 256),
+                                  (1, 64, 64, 2, 9, 256), (1, 64, 64, 2, 0, 256), (1, 64, 64, 0, 1, 0)])
+def test_choice_of_no_such_call(sidon, args):
+    assert sidon._lib.load().sidon_gemm_choice(*args, None, None) == 0
