@@ -2,7 +2,7 @@
 the normalizing blocks) at the sizes where it can go wrong: the shortest chunk,
 frame counts that are no multiple of a block's, one statistics tile and many, a
 chunk that starts off a 16-byte boundary, and frames whose quiet bins lie far
-below their loud ones (needs an MI355X)."""
+below their loud ones; and its parts as calls of their own (needs an MI355X)."""
 
 from __future__ import annotations
 
@@ -30,6 +30,19 @@ def _chunks(batch, samples, valid, seed):
     return out
 
 
+def _check_features(got, host, valid):
+    for b, n in enumerate(valid):
+        want = fo.fbank_exact(host[b, :n])
+        rows = want.shape[0]
+        # log mel is fp32 of a float64 power: 2^-24 x its size (at most 30), over
+        # the bin's deviation, which the normalization divides by
+        logmel = fo.frame_features(np.pad(host[b, :n].astype(np.float64), 160), fo.num_frames(n))
+        dev = np.tile(np.sqrt(logmel.var(axis=0, ddof=1) + fo.VAR_EPS), 2)
+        tol = 16 * 2.0 ** -24 * (30 / dev + np.abs(want))
+        assert (np.abs(got[b, :rows] - want) <= tol).all()
+        assert not got[b, rows:].any()
+
+
 @pytest.mark.parametrize("samples,valid,offset", [
     (640, [640], 0), (640, [400, 641 - 1], 1), (960, [800], 0), (3200, [3200, 1777, 560], 3), (16000, [15999], 0),
     (20480, [20480], 0), (40960, [40959, 30000], 1), (320 * 1300, [320 * 1300 - 77], 2)])
@@ -41,13 +54,41 @@ def test_features_match_float64(sidon, samples, valid, offset):
     fb = sidon.frontend.Fbank(DEV)
     got = fb(chunk, torch.tensor(valid, dtype=torch.int32, device=DEV)).double().cpu().numpy()
     assert got.shape == (len(valid), samples // 320, 160)
-    for b, n in enumerate(valid):
-        want = fo.fbank_exact(host[b, :n])
-        rows = want.shape[0]
-        # log mel is fp32 of a float64 power: 2^-24 x its size (at most 30), over
-        # the bin's deviation, which the normalization divides by
-        logmel = fo.frame_features(np.pad(host[b, :n].astype(np.float64), 160), fo.num_frames(n))
-        dev = np.tile(np.sqrt(logmel.var(axis=0, ddof=1) + fo.VAR_EPS), 2)
-        tol = 16 * 2.0 ** -24 * (30 / dev + np.abs(want))
-        assert (np.abs(got[b, :rows] - want) <= tol).all()
-        assert not got[b, rows:].any()
+    _check_features(got, host, valid)
+
+
+@pytest.mark.parametrize("samples,valid,offset", [
+    (640, [640], 0), (960, [800, 960], 1), (1600, [1600, 1111, 560], 2), (32000, [31999], 3), (32000, [32000, 20001], 0)])
+def test_features_in_parts_match_float64(sidon, samples, valid, offset):
+    """frames, the product with ``frame_transform``, logmel and normalize as calls of
+    their own: the framing exact, the log mel within fp32 of the spectrum it is
+    given, the features as the one call's are held to."""
+    host = _chunks(len(valid), samples, valid, samples + 1)
+    batch, frames = len(valid), samples // 160
+    flat = torch.zeros(host.size + offset, device=DEV)
+    flat[offset:] = torch.from_numpy(host).to(DEV).reshape(-1)
+    fb, lib, stream = sidon.frontend.Fbank(DEV), sidon._lib.load(), torch.cuda.current_stream().cuda_stream
+    rows = torch.full((batch * frames + 1, 400), 7.0, device=DEV)
+    sidon._lib.check("frames", lib.sidon_fbank_frames(flat[offset:].data_ptr(), rows.data_ptr(), batch, samples, stream))
+    padded = torch.nn.functional.pad(torch.from_numpy(host), (160, 160))
+    want = padded.unfold(1, 400, 160)[:, :frames].reshape(batch * frames, 400)
+    assert torch.equal(rows[:-1].cpu(), want) and (rows[-1] == 7).all()
+
+    spec = (rows[:-1].double() @ sidon.frontend.frame_transform().to(DEV).double()).float()
+    logmel = torch.full((batch * frames + 1, 80), 7.0, device=DEV)
+    sidon._lib.check("logmel", lib.sidon_fbank_logmel(
+        spec.data_ptr(), fb.mel_w.data_ptr(), fb.mel_lo.data_ptr(), fb.mel_len.data_ptr(), fb.mel_w.shape[1],
+        logmel.data_ptr(), batch * frames, stream))
+    power = spec[:, :257].double() ** 2 + spec[:, 257:].double() ** 2
+    mel = power.cpu() @ torch.from_numpy(sidon.frontend.mel_banks())
+    want = torch.log(mel.clamp_min(fo.MEL_FLOOR))
+    # a positive sum of up to 16 terms of four roundings each, then the log's
+    assert ((logmel[:-1].double().cpu() - want).abs() <= 2.0 ** -24 * (24 + 4 * want.abs())).all()
+    assert (logmel[-1] == 7).all()
+
+    nbytes = lib.sidon_fbank_workspace_bytes(batch, frames)
+    work, out = torch.empty(nbytes // 4, device=DEV), torch.empty(batch, frames // 2, 160, device=DEV)
+    lens = torch.tensor(valid, dtype=torch.int32, device=DEV)
+    sidon._lib.check("normalize", lib.sidon_fbank_normalize(
+        logmel.data_ptr(), lens.data_ptr(), work.data_ptr(), nbytes, out.data_ptr(), batch, frames, stream))
+    _check_features(out.double().cpu().numpy(), host, valid)
