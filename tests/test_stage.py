@@ -157,35 +157,23 @@ def test_runtime_call_in_a_capture_leaves_both_usable(sidon):
 
 
 @pytest.mark.gpu
-def test_runtime_calls_from_several_streams_do_not_overlap(sidon):
-    """One runtime called from the default stream and from two others in turn,
-    with no synchronisation between the calls: every result, copied on its own
-    stream, equals the same call made alone."""
-    import sys
-
-    from conftest import GOLDEN
-
-    sys.path.insert(0, str(GOLDEN))
-    from make_encoder_golden import encoder_weights
-
-    dev = torch.device("cuda:0")
-    enc = sidon.encoder.HipEncoder(sidon.encoder.pack_weights(encoder_weights(2, 2, seed=9)), dev)
-    rt = sidon.runtime.EncoderRuntime(enc, max_batch=1, max_seconds=12)
+@pytest.mark.parametrize("use_graph", [True, False])
+@pytest.mark.parametrize("first,second", [(0, 1), (1, 0), (1, 2)])
+def test_runtime_call_waits_for_the_one_before(sidon, use_graph, first, second):
+    """A long call on one stream (0: the default one) and at once a short one on
+    another, nothing between them: the short one, which shares the long one's
+    buffers, equals the same call made alone."""
+    rt = _runtime(sidon, 96, use_graph=use_graph)
     gen = torch.Generator().manual_seed(1)
-    feats = [torch.randn(1, n, 160, generator=gen).to(dev) for n in (480, 301, 480, 97, 600, 599)]
-    alone = []
-    for f in feats:
-        alone.append(rt.run(f).clone())
+    long, short = (torch.randn(1, n, 160, generator=gen).cuda() for n in (4800, 97))
+    rt.run(long)
+    alone = rt.run(short).clone()
+    streams = [torch.cuda.default_stream(), torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for _ in range(3):
+        with torch.cuda.stream(streams[first]):
+            rt.run(long)
+        with torch.cuda.stream(streams[second]):
+            got = rt.run(short).clone()
         torch.cuda.synchronize()
-    streams = [torch.cuda.current_stream(dev), torch.cuda.Stream(dev), torch.cuda.Stream(dev)]
-    for rep in range(3):
-        got = []
-        for i, f in enumerate(feats):
-            with torch.cuda.stream(streams[(i + rep) % 3]):
-                got.append(rt.run(f).clone())
-                # the next call may start as soon as this one's buffer is read
-                for s in streams:
-                    s.wait_stream(streams[(i + rep) % 3])
-        torch.cuda.synchronize()
-        for a, b in zip(got, alone):
-            assert torch.equal(a, b), rep
+        assert torch.equal(got, alone)
