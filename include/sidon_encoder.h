@@ -324,7 +324,7 @@ int sidon_fbank_normalize(const float* logmel, const int* valid, float* workspac
 /*
  * sidon_fbank_normalize without a workspace argument: the same kernels and
  * results (bit for bit), with the statistics held in a static device array
- * of the library (1.9 MiB per device, kept until the process ends) instead
+ * of the library (1.3 MiB per device, kept until the process ends) instead
  * of caller memory.  No counterpart in the reference: it is for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops).  It allocates nothing and calls no allocating routine.  B <= 32

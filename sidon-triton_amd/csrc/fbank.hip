@@ -42,6 +42,7 @@ constexpr int kLmThreads = 256;      // logmel: threads per block (kMel * kLmLan
 constexpr int kLanes = 4;            // normalize: frame lanes x 80 bins per block
 constexpr int kApplyFrames = 32;     // normalize: frames per apply block
 constexpr int kMaxTiles = 64;
+constexpr int kTileFloats = 2 * kMel;  // a statistics tile in the workspace: means, squared deviations
 constexpr int kStatsCache = 40;      // statistics: frames per lane held in registers
 constexpr int kSpWaves = 4;          // spectrum: wavefronts per block
 // Frames per wavefront and block: with 8 per block a 96 s chunk's 1200 blocks
@@ -372,7 +373,7 @@ __global__ void __launch_bounds__(kLanes * kMel) stats_kernel(const float* __res
   red[fl][m] = q;
   __syncthreads();
   if (fl == 0) {
-    float* dst = part + ((int64_t)b * G + g) * 2 * kMel + m;
+    float* dst = part + ((int64_t)b * G + g) * kTileFloats + m;
     dst[0] = mean;
     dst[kMel] = (red[0][m] + red[1][m]) + (red[2][m] + red[3][m]);
   }
@@ -424,7 +425,7 @@ __global__ void __launch_bounds__(kLanes * kMel) apply_kernel(const float* __res
 #pragma unroll
   for (int j = 0; j < kOwn; ++j) {
     const int g = kOwn * fl + j;
-    const float* src = part + ((int64_t)b * G + min(g, G - 1)) * 2 * kMel + m;  // no branch between the loads
+    const float* src = part + ((int64_t)b * G + min(g, G - 1)) * kTileFloats + m;  // no branch between the loads
     own[j] = Moments{g < G ? (float)max(min(per, tf - g * per), 0) : 0.f, src[0], g < G ? src[kMel] : 0.f};
   }
 #pragma unroll
@@ -449,11 +450,11 @@ int tiles_for(int F) { return F / 128 < 1 ? 1 : (F / 128 > kMaxTiles ? kMaxTiles
 
 // Scratch of sidon_fbank_normalize_noalloc: the normalize workspace of up
 // to kScratchItems items of any length (tiles_for() caps the tiles at
-// kMaxTiles), 1.9 MiB in all, one copy per device for the life of the
+// kMaxTiles), 1.3 MiB in all, one copy per device for the life of the
 // process.  Every word a call reads was written earlier in the same call, so
 // nothing needs clearing between calls.
 constexpr int kScratchItems = 32;
-constexpr size_t kScratchFloats = (size_t)kScratchItems * (kMaxTiles * kMel * 3 + kMel * 2);
+constexpr size_t kScratchFloats = (size_t)kScratchItems * kMaxTiles * kTileFloats;
 static __device__ __align__(256) float scratch[kScratchFloats];
 
 // Device address of `scratch` per device, taken once per device with that
@@ -553,7 +554,7 @@ SIDON_API int sidon_fbank_features(const float* chunk, const int* valid, const d
 
 SIDON_API size_t sidon_fbank_workspace_bytes(int B, int F) {
   if (B < 1 || F < 1) return 0;
-  return (size_t)B * (tiles_for(F) * kMel * 3 + kMel * 2) * sizeof(float);
+  return (size_t)B * tiles_for(F) * kTileFloats * sizeof(float);
 }
 
 SIDON_API int sidon_fbank_normalize(const float* logmel, const int* valid, float* workspace, size_t workspace_bytes,

@@ -87,8 +87,9 @@ def test_features_in_parts_match_float64(sidon, samples, valid, offset):
     assert (logmel[-1] == 7).all()
 
     nbytes = lib.sidon_fbank_workspace_bytes(batch, frames)
-    work, out = torch.empty(nbytes // 4, device=DEV), torch.empty(batch, frames // 2, 160, device=DEV)
+    work, out = torch.full((nbytes // 4 + 64,), 7.0, device=DEV), torch.empty(batch, frames // 2, 160, device=DEV)
     lens = torch.tensor(valid, dtype=torch.int32, device=DEV)
     sidon._lib.check("normalize", lib.sidon_fbank_normalize(
         logmel.data_ptr(), lens.data_ptr(), work.data_ptr(), nbytes, out.data_ptr(), batch, frames, stream))
+    assert (work[-64:] == 7).all()
     _check_features(out.double().cpu().numpy(), host, valid)
