@@ -80,8 +80,10 @@ int sidon_silu(void* h, int64_t n, sidon_stream_t stream);
  * sidon_gemm_bias_act_fits(M, N, K) says whether a shape is supported (pure
  * host function); sidon_gemm_bias_act_preferred(M, N, K) whether the kernel
  * is expected to beat a library GEMM followed by sidon_silu on the current
- * device, and sidon_gemm_lt_act (its 320 x 256 tiles keep >= 4/5 of the CUs
- * busy in every round).  Neither has a counterpart in the reference.
+ * device, and sidon_gemm_lt_act (past that one's own kernel, where 320 x 256
+ * tiles would keep >= 4/5 of the CUs busy in every round; N = 4096, K = 1024:
+ * from 3841 rows on, 10% slower up to 4096).  Neither has a counterpart in
+ * the reference.
  */
 int sidon_gemm_bias_act_fits(int M, int N, int K);
 int sidon_gemm_bias_act_preferred(int M, int N, int K);
@@ -192,11 +194,13 @@ int sidon_gemm_choice(int M, int N, int K, int epilogue, int max_splits, int cus
  * x [M, K] and w [N, K] row-major with row strides ldx, ldw >= K (K
  * contiguous); y [M, N] row-major with row stride ldy >= N.  dtype 0: fp32
  * x, w, y; 1: fp16 x, w, y (beta must be 0); 2: fp16 x, w and fp32 y.
- * Used for the pointwise conv's first F.linear of the encoder
- * (src/sidon_triton/triton_encoder.py:504; dtype 1) and the framing matmul
- * of the front end (src/sidon_triton/frontend.py:222; dtype 0).  dtype 2
- * with beta 1 is the form of the residual projections of res() (:491-492),
- * which the encoder keeps on torch.addmm.
+ * The encoder uses it for the pointwise conv's first F.linear
+ * (src/sidon_triton/triton_encoder.py:504; dtype 1) where sidon_gemm_glu does
+ * not take the width or layout.  dtype 0 is the form of the front end's
+ * framing matmul (src/sidon_triton/frontend.py:222) for a caller of the
+ * front end's parts, dtype 2 with beta 1 that of the residual projections of
+ * res() (:491-492), which run on sidon_gemm_res / sidon_gemm_part or on
+ * torch.addmm.
  *
  * sidon_gemm_nt runs the kernel recorded for the problem (shape, strides,
  * dtype, beta != 0) by sidon_gemm_nt_tune or sidon_gemm_nt_pin, else

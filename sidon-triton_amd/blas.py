@@ -1,11 +1,12 @@
-"""Plain GEMMs of the encoder and the front end on rocBLAS (csrc/blas.hip).
+"""Plain GEMMs on rocBLAS (csrc/blas.hip).
 
 ``gemm_nt(x, w, out, beta=0.0)`` computes ``out = x . w^T + beta * out`` for
 row-major x [M, K] and w [N, K] (rows K-contiguous) with fp32 sums, in three
 type combinations:
 
-  * fp32 x, w, out -- the framing matmul of the front end
-    (src/sidon_triton/frontend.py:222);
+  * fp32 x, w, out -- the form of the framing matmul of the reference's front
+    end (src/sidon_triton/frontend.py:222), for a caller who takes the front end
+    in parts (``frontend.Fbank`` transforms its frames itself);
   * fp16 x, w, out (beta 0) -- the pointwise conv's first F.linear
     (src/sidon_triton/triton_encoder.py:504) at widths that
     ``conformer.linear_glu`` does not take;
@@ -13,7 +14,7 @@ type combinations:
     of res(), ``torch.addmm(x, a, W^T, out_dtype=float32, out=x)`` (:491-492).
     The encoder does not use rocBLAS for those: they run on this library's
     tiled kernel (``conformer.residual_partials`` / ``residual_gemm``), which
-    measured faster.
+    measured faster, or past 5 M outputs on torch.addmm.
 
 The first call of a problem (shape, strides, types, beta != 0) on a device,
 made while the stream is not capturing, times rocBLAS's kernels for it on

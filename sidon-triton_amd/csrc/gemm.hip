@@ -29,8 +29,8 @@
 //   4096 x 1024 + bias + SiLU    7.5 | 12.0+  12.3 | 14.3+ 20.4 | 22.3+ 47.0 | 47.0+  (library without SiLU)
 //   3072 x 1024 + bias           6.2 |  9.7    9.7 | 12.8  15.0 | 17.7  35.4 | 30.9
 //   2048 x 1024 + GLU            5.3 |  8.6+   6.8 |  9.7+ 10.3 | 13.2+ 23.3 | 30.6+  (library without GLU)
-//   1024 x 4096 fp32, split K    6.2 | 12.2   12.3 | 20.8  20.4 | 28.8  45.1 | 50.6
-//   1024 x 1024 fp32, split K    4.0 |  8.2    5.6 |  9.2   7.8 | 11.0  14.6 | 19.1
+//   1024 x 4096 fp32, split K    6.9 | 12.3   12.3 | 20.8  19.7 | 27.5  45.4 | 48.7 (4800: in place)
+//   1024 x 1024 fp32             4.0 |  8.1    6.1 |  9.0   8.0 | 11.0  17.3 | 18.4 (split at 150, else in place)
 #include "gemm_tile.h"
 
 #include "sidon_encoder.h"
@@ -221,10 +221,11 @@ SIDON_API int sidon_gemm_bias_act_fits(int M, int N, int K) {
   return M >= 1 && N >= 256 && N % 256 == 0 && K >= 64 && K % 64 == 0 ? 1 : 0;
 }
 
-// Against the library with the SiLU in its epilogue this pays off past
-// gemm_half_preferred's range where 320 x 256 tiles, one per CU, keep four
-// fifths of the CUs busy in every round (M x 4096 x 1024: 4200 45.9 against
-// 56.7 us, 4800 47.0 against 47.0 without its SiLU; 3600, 192 tiles, 40 against 32.5).
+// Past gemm_half_preferred's range, where 320 x 256 tiles would keep four fifths
+// of the CUs busy in every round (the tile that then runs is the cost rule's: 256 x
+// 256 up to 4096 rows).  M x 4096 x 1024, us, own | the library with the SiLU in
+// its epilogue: 3400 35.0 | 32.2, 3700 36.3 | 34.2, 4097 42.3 | 47.3, 4200 43.7 | 63.0,
+// 4800 46.1 | 50.4.  From 3841 to 4096 rows the line is generous (37.5 | 33.9).
 SIDON_API int sidon_gemm_bias_act_preferred(int M, int N, int K) {
   if (!sidon_gemm_bias_act_fits(M, N, K)) return 0;
   if (sidon::check_device() != SIDON_OK) return 0;

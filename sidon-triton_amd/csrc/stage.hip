@@ -5,8 +5,8 @@
 //
 // The lengths travel as kernel arguments.  As a copy from host memory they
 // made the host wait for the previous call's graph, so every call paid its
-// launches (60 us) with the GPU idle; the data copy is bound by HBM (31 MB
-// at most per item) and far below that.
+// launches (60 us) with the GPU idle; the data copy is bound by HBM (a 96 s item
+// is 6 MB of samples or 3 MB of features, read and written) and far below that.
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>

@@ -71,11 +71,12 @@ def bucket_samples(samples: int, max_samples: int) -> int:
 
 def stage_items(src: torch.Tensor, counts, dst: torch.Tensor, outs) -> None:
     """dst[b] = src[b, :counts[b]] and zeros after it, and for each (out, values)
-    of ``outs`` (at most two) out[b] = values[b], on the current stream without
-    waiting for its earlier work.  src [B, ...] (any device and type), dst [B, ...] fp32
-    contiguous on the device, out int32 [B] on the device, values host ints.
-    One launch when src is a contiguous fp32 tensor of dst's device; a host src
-    is copied before the call returns, so the caller may overwrite it."""
+    of ``outs`` (at most two) out[b] = values[b], on the current stream.  src
+    [B, ...] (any device and type), dst [B, ...] fp32 contiguous on the device, out
+    int32 [B] on the device, values host ints.  One launch, enqueued without
+    waiting for the stream's earlier work, when src is a contiguous fp32 tensor
+    of dst's device; a host src is copied before the call returns, so the caller
+    may overwrite it, and that copy does wait for the stream."""
     batch = dst.shape[0]
     n, m = src[0].numel(), dst[0].numel()
     direct = src.device == dst.device and src.dtype == torch.float32 and src.is_contiguous() and m % 4 == 0

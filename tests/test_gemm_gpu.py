@@ -1,7 +1,7 @@
 """The fused feed-forward input projection (GEMM + bias + SiLU, csrc/gemm.hip;
 hipBLASLt with the bias and SiLU in its epilogue, csrc/blaslt.hip) against
 float32 torch and against hipBLASLt followed by the in-place SiLU, and the
-residual GEMM (csrc/gemm_res.hip) (needs an MI355X)."""
+residual GEMM (csrc/gemm.hip) (needs an MI355X)."""
 
 from __future__ import annotations
 
@@ -236,7 +236,7 @@ def test_runtime_full_chunk_graph_replays_match_eager(sidon):
     assert len(rt.graphs) == 1
 
 
-# ---- the residual projection into the fp32 stream (csrc/gemm_res.hip) ----
+# ---- the residual projection into the fp32 stream (csrc/gemm.hip) ----
 
 @pytest.mark.parametrize("m,n,k,ldx,ldy", [
     (750, 1024, 4096, None, None),
