@@ -105,7 +105,7 @@ int sidon_gemm_bias_act(const void* x, int ldx, const void* w, int ldw, const vo
  * src/sidon_triton/triton_encoder.py:498-499 and :507-508.  Shapes: M, N,
  * K >= 1, strides >= the row lengths, every operand 2-byte aligned.  Where
  * sidon_gemm_half_preferred(M, N, K) (N and K multiples of 64, up to 9 * 2^20
- * outputs) and the operands are 16-byte aligned (the bias 8-byte) with strides
+ * outputs, but more than 2^18 where K > 2048) and the operands are 16-byte aligned (the bias 8-byte) with strides
  * that are multiples of 8, x and w each span less than 4 GiB and y lies apart
  * from them, this library's own kernel runs with the same rounding;
  * sidon_gemm_half_takes says so for a call's operands (pure host function).

@@ -10,9 +10,10 @@
 // terms this is y^T = op(w) . x^T with op = transpose, the bias one value per
 // row of y^T.
 //
-// Problems of up to 9 M outputs whose shape and alignment this library's tiled
-// GEMM kernel takes run on it instead (gemm.hip, the same rounding; 12.0 -> 7.5
-// us at 150 x 4096 x 1024, 22.3 -> 20.4 at M = 1600); the rest stay here.
+// Problems of up to 9 M outputs (few ones only of a K up to 2048) whose shape
+// and alignment this library's tiled GEMM kernel takes run on it instead
+// (gemm.hip, the same rounding; 12.0 -> 7.5 us at 150 x 4096 x 1024, 22.3 -> 20.4
+// at M = 1600); the rest stay here.
 //
 // The kernel is hipBLASLt's first heuristic choice for the problem with no
 // workspace (no split-K partials: a call shares no memory with other calls

@@ -180,6 +180,14 @@ bool overlaps(const void* x, int ldx, const void* w, int ldw, const void* y, int
   return (xb < ye && yb < xe) || (wb < ye && yb < we);
 }
 
+// Few outputs of a long K: a handful of workgroups that walk all of it, where the
+// library's kernels are faster (us, this kernel | library: fp16 with SiLU 150 x 256
+// x 4096 11.7 | 8.3, 150 x 1024 x 4096 15.2 | 12.3, x 8192 26.3 | 20.2, but 400 x
+// 1024 x 4096 level; in place 1024 x 4096 150 rows 15.0 | 12.3, 225 13.3 | 12.1, 257
+// 13.5 | 14.9; 512 x 4096 400 rows 13.0 | 11.3; 2048 x 4096 100 rows 13.7 | 12.7, 200
+// 14.1 | 14.4; at K = 2048 this one is ahead from 25 rows on, 8.2 | 9.7 at 150 x 1024).
+bool few_of_long_k(int M, int N, int K) { return (int64_t)M * N <= 1 << 18 && K > 2048; }
+
 }  // namespace
 
 namespace sidon {
@@ -189,7 +197,8 @@ namespace sidon {
 // against 30.8 us, 3600 30.5 against 27.6; M x 4096: 2000 23.0 against 24.1
 // without its SiLU, 3000 32.9 against 28.7).
 bool gemm_half_preferred(int M, int N, int K) {
-  return M >= 1 && N >= 64 && N % 64 == 0 && K >= 64 && K % 64 == 0 && (int64_t)M * N <= (int64_t)9 << 20;
+  return M >= 1 && N >= 64 && N % 64 == 0 && K >= 64 && K % 64 == 0 && (int64_t)M * N <= (int64_t)9 << 20 &&
+         !few_of_long_k(M, N, K);
 }
 
 bool gemm_half_takes(const void* x, int ldx, const void* w, int ldw, const void* bias, const void* y, int ldy, int M,
@@ -289,15 +298,11 @@ SIDON_API int sidon_gemm_glu(const void* x, int ldx, const void* w, int ldw, voi
 
 SIDON_API int sidon_gemm_res_fits(int M, int N, int K) { return res_fits(M, N, K) ? 1 : 0; }
 
-// The library's kernels were slower at the encoder's two residual shapes up to
-// 4800 rows of N = 1024, except at few outputs of a long K, where they split K
-// (us, in place | library: 1024 x 4096 150 rows 15.0 | 12.3, 225 13.3 | 12.1, 257
-// 13.5 | 14.9, x 2048 150 rows 8.2 | 9.7; 512 x 4096 400 rows 13.0 | 11.3; 2048 x
-// 4096 100 rows 13.7 | 12.7, 200 14.1 | 14.4).  Past the measured range they are
-// kept.
+// Past few outputs of a long K the library's kernels were slower at the encoder's
+// two residual shapes up to 4800 rows of N = 1024; past the measured range they
+// are kept.
 SIDON_API int sidon_gemm_res_preferred(int M, int N, int K) {
-  const int64_t outputs = (int64_t)M * N;
-  if (!res_fits(M, N, K) || outputs > (int64_t)5 << 20 || (outputs <= 1 << 18 && K > 2048)) return 0;
+  if (!res_fits(M, N, K) || (int64_t)M * N > (int64_t)5 << 20 || few_of_long_k(M, N, K)) return 0;
   return sidon::check_device() == SIDON_OK ? 1 : 0;
 }
 

@@ -43,13 +43,15 @@ def test_projection_takes_only_what_the_kernel_reads(sidon, over):
     """The answer that sends a call to the tiled kernel: each case wrong in one
     argument (sizes, strides, alignment of each operand and of the bias, spans of
     4 GiB, an output over an operand); the plain call, an 8-byte bias and touching
-    ranges are taken."""
+    ranges are taken, few outputs only of a K up to 2048."""
     def takes(**over):
         a = dict(x=1 << 40, ldx=1024, w=1 << 41, ldw=1024, bias=1 << 43, y=1 << 42, ldy=3072, M=750, N=3072, K=1024)
         a.update(over)
         return sidon._lib.load().sidon_gemm_half_takes(a["x"], a["ldx"], a["w"], a["ldw"], a["bias"], a["y"],
                                                        a["ldy"], a["M"], a["N"], a["K"])
 
+    assert takes(K=2048, ldx=2048, ldw=2048) == takes(M=86, K=4096, ldx=4096, ldw=4096) == 1
+    assert takes(M=85, K=4096, ldx=4096, ldw=4096) == takes(M=85, K=2112, ldx=2112, ldw=2112) == 0
     assert takes() == takes(bias=(1 << 43) + 8) == takes(bias=None) == takes(y=(1 << 40) + 750 * 2048) == 1
     assert takes(**over) == 0
 
