@@ -183,6 +183,10 @@ __device__ __forceinline__ void radix4(Complex (&v)[4]) {
   v[3] = {b.x - d.y, b.y + d.x};
 }
 
+__device__ __forceinline__ float power_of(Complex a, bool infinite) {
+  return infinite ? __builtin_inff() : (float)fma(a.x, a.x, a.y * a.y);
+}
+
 // LDS position of point i: one spare point per 16 spreads the strided writes.
 __device__ __forceinline__ int spread(int i) { return i + (i >> 4); }
 
@@ -245,12 +249,17 @@ __global__ void __launch_bounds__(64 * kSpWaves) spectrum_kernel(const float* __
 
   Complex* own = points[w];
   Complex v[kSpFrames][4];
+  // An infinite sample makes every power infinite, and so the item's features NaN,
+  // as in a product with the transform matrix; the FFT alone gives NaN powers, which
+  // the floor of the log would take for silence.
+  bool infinite[kSpFrames];
 #pragma unroll
   for (int q = 0; q < kSpFrames; ++q) {
     double s = 0.;
 #pragma unroll
     for (int r = 0; r < 4; ++r) s += (double)in[q][r][1] + (double)in[q][r][2];
     const double mean = sidon::wave_sum(s) * (1. / kFrameSize);
+    infinite[q] = __builtin_isinf(mean);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const double before = in[q][r][0] - mean, x0 = in[q][r][1] - mean, x1 = in[q][r][2] - mean;
@@ -296,10 +305,10 @@ __global__ void __launch_bounds__(64 * kSpWaves) spectrum_kernel(const float* __
       const Complex e = {0.5 * (z.x + c.x), 0.5 * (z.y - c.y)}, o = {0.5 * (z.x - c.x), 0.5 * (z.y + c.y)};
       const Complex u = cmul(o, root[r]);
       const Complex lo = {e.x + u.y, e.y - u.x}, hi = {e.x - u.y, e.y + u.x};
-      dst[lane + 64 * r] = (float)fma(lo.x, lo.x, lo.y * lo.y);
-      dst[kPoints - lane - 64 * r] = (float)fma(hi.x, hi.x, hi.y * hi.y);
+      dst[lane + 64 * r] = power_of(lo, infinite[q]);
+      dst[kPoints - lane - 64 * r] = power_of(hi, infinite[q]);
     }
-    if (lane == 0) dst[128] = (float)fma(v[q][2].x, v[q][2].x, v[q][2].y * v[q][2].y);
+    if (lane == 0) dst[128] = power_of(v[q][2], infinite[q]);
   }
   __syncthreads();
   mel_log<kSpBlock, kSpLanes>(power, mel_w, mel_lo, mel_len, max_len, out, f0, R);

@@ -57,6 +57,22 @@ def test_features_match_float64(sidon, samples, valid, offset):
     _check_features(got, host, valid)
 
 
+@pytest.mark.parametrize("at", [0, 159, 5000, 5001, 14999])
+@pytest.mark.parametrize("values", [[float("inf")], [float("-inf")], [float("inf")] * 3, [3e38]])
+def test_an_infinite_sample_shows_in_its_item_alone(sidon, at, values):
+    """Infinite, or too large for an fp32 power: its item's features are NaN (as
+    float64 torch gives them), the other item's the same bits as without it."""
+    host = torch.from_numpy(_chunks(2, 16000, [15000, 15000], 9)).to(DEV)
+    lens = torch.tensor([15000, 15000], dtype=torch.int32, device=DEV)
+    fb = sidon.frontend.Fbank(DEV)
+    want = fb(host, lens)
+    assert torch.isfinite(want).all()
+    host[0, at:min(at + len(values), 15000)] = torch.tensor(values, device=DEV)[:15000 - at]
+    got, frames = fb(host, lens), fo.num_frames(15000)
+    assert got[0].reshape(-1, 80)[:frames].isnan().all() and torch.equal(got[1], want[1])
+    assert torch.equal(got[0].reshape(-1, 80)[frames:], want[0].reshape(-1, 80)[frames:])
+
+
 @pytest.mark.parametrize("samples,valid,offset", [
     (640, [640], 0), (960, [800, 960], 1), (1600, [1600, 1111, 560], 2), (32000, [31999], 3), (32000, [32000, 20001], 0)])
 def test_features_in_parts_match_float64(sidon, samples, valid, offset):
