@@ -147,9 +147,8 @@ int sidon_gemm_glu(const void* x, int ldx, const void* w, int ldw, void* y, int 
  * >= N; x, w, y 16-byte aligned; x and w must not overlap y (checked on the byte ranges
  * the call touches: SIDON_E_SHAPE).  sidon_gemm_res_fits(M, N, K) says whether
  * a shape is supported (pure host function); sidon_gemm_res_preferred(M, N,
- * K) whether it is expected to beat a library GEMM on the current device (up
- * to 5 * 2^20 outputs, but more than 2^18 where K > 2048).  Neither has a
- * counterpart in the reference.
+ * K) whether a call of its own is expected to beat torch.addmm on the current
+ * device (up to 5 * 2^20 outputs).  Neither has a counterpart in the reference.
  */
 int sidon_gemm_res_fits(int M, int N, int K);
 int sidon_gemm_res_preferred(int M, int N, int K);

@@ -181,11 +181,8 @@ bool overlaps(const void* x, int ldx, const void* w, int ldw, const void* y, int
 }
 
 // Few outputs of a long K: a handful of workgroups that walk all of it, where the
-// library's kernels are faster (us, this kernel | library: fp16 with SiLU 150 x 256
-// x 4096 11.7 | 8.3, 150 x 1024 x 4096 15.2 | 12.3, x 8192 26.3 | 20.2, but 400 x
-// 1024 x 4096 level; in place 1024 x 4096 150 rows 15.0 | 12.3, 225 13.3 | 12.1, 257
-// 13.5 | 14.9; 512 x 4096 400 rows 13.0 | 11.3; 2048 x 4096 100 rows 13.7 | 12.7, 200
-// 14.1 | 14.4; at K = 2048 this one is ahead from 25 rows on, 8.2 | 9.7 at 150 x 1024).
+// library's kernels are faster (us, this kernel | library: 150 x 256 x 4096 11.7 |
+// 8.3, 150 x 1024 x 4096 15.2 | 12.3, x 8192 26.3 | 20.2, but 400 x 1024 x 4096 level).
 bool few_of_long_k(int M, int N, int K) { return (int64_t)M * N <= 1 << 18 && K > 2048; }
 
 }  // namespace
@@ -298,11 +295,14 @@ SIDON_API int sidon_gemm_glu(const void* x, int ldx, const void* w, int ldw, voi
 
 SIDON_API int sidon_gemm_res_fits(int M, int N, int K) { return res_fits(M, N, K) ? 1 : 0; }
 
-// Past few outputs of a long K the library's kernels were slower at the encoder's
-// two residual shapes up to 4800 rows of N = 1024; past the measured range they
-// are kept.
+// The library's kernels were slower at the encoder's two residual shapes up to
+// 4800 rows of N = 1024, but for few outputs of a long K (1024 x 4096, us, in place |
+// library: 150 rows 15.0 | 12.3, 225 13.3 | 12.1, 257 13.5 | 14.9).  There torch.addmm's
+// host side outweighs that for a call launched on its own (a feed-forward step of
+// 150 rows, 30.2 us a pass against 42.2; in a graph 25 against 22.4), and a caller with
+// a buffer splits K.  Past the measured range the library is kept.
 SIDON_API int sidon_gemm_res_preferred(int M, int N, int K) {
-  if (!res_fits(M, N, K) || (int64_t)M * N > (int64_t)5 << 20 || few_of_long_k(M, N, K)) return 0;
+  if (!res_fits(M, N, K) || (int64_t)M * N > (int64_t)5 << 20) return 0;
   return sidon::check_device() == SIDON_OK ? 1 : 0;
 }
 

@@ -259,12 +259,11 @@ def test_residual_projections_take_no_memory(sidon, rows):
 
 
 @pytest.mark.parametrize("rows,n,k,in_place,split", [
-    (150, 1024, 4096, 0, True), (256, 1024, 4096, 0, True), (257, 1024, 4096, 1, True), (150, 1024, 2048, 1, True),
-    (512, 512, 4096, 0, True), (513, 512, 4096, 1, True), (25, 1024, 1024, 1, True), (5120, 1024, 1024, 1, False),
-    (5121, 1024, 1024, 0, False), (100, 1024, 192, 0, False)])
+    (150, 1024, 4096, 1, True), (512, 512, 4096, 1, True), (150, 1024, 2048, 1, True), (25, 1024, 1024, 1, True),
+    (5120, 1024, 1024, 1, False), (5121, 1024, 1024, 0, False), (100, 1024, 192, 0, False)])
 def test_residual_route(sidon, rows, n, k, in_place, split):
-    """Split where a buffer is there and the cost rule splits, else in place where
-    that is the faster one, else the library."""
+    """Split where a buffer is there and the cost rule splits, else in place up to
+    5 * 2^20 outputs, else the library."""
     ops = sidon.conformer
     assert ops.residual_gemm_preferred(rows, n, k, DEV) == bool(in_place)
     assert ops.residual_splits(rows, n, k, DEV, part=False) == in_place
