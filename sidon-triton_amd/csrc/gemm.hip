@@ -299,7 +299,7 @@ SIDON_API int sidon_gemm_res_fits(int M, int N, int K) { return res_fits(M, N, K
 // 4800 rows of N = 1024, but for few outputs of a long K (1024 x 4096, us, in place |
 // library: 150 rows 15.0 | 12.3, 225 13.3 | 12.1, 257 13.5 | 14.9).  There torch.addmm's
 // host side outweighs that for a call launched on its own (a feed-forward step of
-// 150 rows, 30.2 us a pass against 42.2; in a graph 25 against 22.4), and a caller with
+// 150 rows, 32.0 us a pass against 42.2; in a graph 24.0 against 22.4), and a caller with
 // a buffer splits K.  Past the measured range the library is kept.
 SIDON_API int sidon_gemm_res_preferred(int M, int N, int K) {
   if (!res_fits(M, N, K) || (int64_t)M * N > (int64_t)5 << 20) return 0;
